@@ -1,4 +1,4 @@
-// q8_gemv.hip -- decode-path Q8 GEMV for gfx950 (f32 activations, s <= 4 per pass).
+// q8_gemv.hip -- decode-path Q8 GEMV for gfx950 (one row of f32 activations).
 //
 // y[b, j] = sum_g scale[j, g] * sum_{k in g} x[b, k] * q[j, k]
 // (k_mm_q8, src/llama_q8.mojo:54-93: unscaled dot per group, then one scale
@@ -25,7 +25,9 @@
 // Rows are distributed over a grid sized to fill all 256 CUs; workgroups
 // stride over row tiles, so a large matrix (lm_head) is one launch.
 //
-// A generic fallback handles packed rows or x that are not 16-byte aligned.
+// Packed rows or x that are not 16-byte aligned take the same kernel with
+// loads of 2- and 4-byte alignment (1600 -> 4800 13.4 -> 4.8 us and 11008 ->
+// 4096 85.9 -> 11.4 us against one code per lane and load).
 #include "q8_device.h"
 #include "q8_launch.h"
 
@@ -50,8 +52,24 @@ __host__ __device__ constexpr int64_t xs_index(int64_t i) { return (i >> 4) * 20
 __host__ __device__ constexpr int64_t xs_floats(int64_t n) { return (n + 15) / 16 * 20; }
 constexpr bool x_padded(int pre, int post) { return !(pre == PRE_NONE && post == POST_STORE); }
 
+// 16 bytes of a packed row and 4 floats of x at the alignment the call has:
+// 16 bytes, or with UA the 2 and 4 bytes that every call has (still one
+// load instruction; the hardware splits those that straddle a line).
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+template <bool UA>
+__device__ __forceinline__ u32x4 stream16(const uint8_t *p) {
+  if constexpr (UA) return __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2 *>(p));
+  else return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+}
+template <bool UA>
+__device__ __forceinline__ f32x4 load_f4(const float *p) {
+  if constexpr (UA) return *reinterpret_cast<const f32x4_a4 *>(p);
+  else return *reinterpret_cast<const f32x4 *>(p);
+}
+
 template <int G, int KIND, int S, int R, int SPLITK, bool XLDS, int PRE = PRE_NONE,
-          int POST = POST_STORE, int NPF = 1, int NW = kWaves>
+          int POST = POST_STORE, int NPF = 1, int NW = kWaves, bool UA = false>
 __global__ __launch_bounds__(64 * NW) void gemv_kernel(
     const uint8_t *__restrict__ w, int64_t row_bytes, int64_t n,
     const float *__restrict__ x, int64_t m, float *y, const uint16_t *__restrict__ wn,
@@ -118,8 +136,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
       const int64_t k = kc + 1024 * p < k_hi ? kc + 1024 * p : base;
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        q[p][r] = __builtin_nontemporal_load(
-            reinterpret_cast<const u32x4 *>(rowp[r] + scale_bytes + k));
+        q[p][r] = stream16<UA>(rowp[r] + scale_bytes + k);
 #pragma unroll
       for (int r = 0; r < R; ++r) sc[p][r] = load_scale<KIND>(rowp[r], k / G);
     }
@@ -145,7 +162,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
     for (int u = 0; u < XB; ++u) {
       const int64_t i = i0 + 4 * NT * u;
       if (i < tot) {
-        xv[u] = *reinterpret_cast<const f32x4 *>(x + i);
+        xv[u] = load_f4<UA>(x + i);
         if constexpr (PRE == PRE_SWIGLU) uv[u] = *reinterpret_cast<const f32x4 *>(x + m + i);
         if constexpr (PRE == PRE_RMSNORM) wb[u] = *reinterpret_cast<const uint2 *>(wn + i);
       }
@@ -157,9 +174,8 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
 #pragma unroll
     for (int p = 0; p < NPF; ++p) {
       const int64_t k = k_first + 1024 * p < k_hi ? k_first + 1024 * p : base;
-      const f32x4 *xv4 = reinterpret_cast<const f32x4 *>(x + k);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) xr[p][c] = xv4[c];
+      for (int c = 0; c < 4; ++c) xr[p][c] = load_f4<UA>(x + k + 4 * c);
     }
   }
   load_chunk(rowp, k_first);
@@ -284,12 +300,12 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
           xc = xr[XREG ? p : 0][2];
           xd = xr[XREG ? p : 0][3];
         } else {
-          const f32x4 *xv4 = reinterpret_cast<const f32x4 *>(
-              xp + (XPAD ? xs_index(b * m + kx) : b * m + kx));
-          xa = xv4[0];
-          xb = xv4[1];
-          xc = xv4[2];
-          xd = xv4[3];
+          // (staged x is aligned whatever the call's x is)
+          const float *xq = xp + (XPAD ? xs_index(b * m + kx) : b * m + kx);
+          xa = load_f4<UA && !XLDS>(xq);
+          xb = load_f4<UA && !XLDS>(xq + 4);
+          xc = load_f4<UA && !XLDS>(xq + 8);
+          xd = load_f4<UA && !XLDS>(xq + 12);
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -403,8 +419,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
   }
 }
 
-// Any alignment and either activation dtype: one wavefront per output,
-// one code per lane per step.
+// Any alignment, row count and activation dtype: one wavefront per output,
+// one code per lane per step.  Only for rows too long for the fragment
+// scratch of the MFMA path (launch_mid).
 template <int G, int KIND, bool XBF16>
 __global__ __launch_bounds__(256) void gemv_generic_kernel(
     const uint8_t *__restrict__ w, int64_t row_bytes, int64_t n,
@@ -441,18 +458,14 @@ int grid_for(int64_t tiles, int64_t cap) {
   return (int)(tiles < cap ? (tiles > 0 ? tiles : 1) : cap);
 }
 
-// NPF: K steps in flight per wave.  Batches of 2-4 rows (the unaligned
-// fallback) keep one step for waves of 2+ rows (registers against
-// occupancy).  One activation row puts the wave's whole K range in flight,
+// NPF: K steps in flight per wave.  A wave puts its whole K range in flight,
 // up to 4 steps (2 or 4, by the range): every wave waits on memory once, so
 // the weights stream at full rate from the start instead of in two waves of
 // requests (gate|up 2048 -> 16384: first step's data in 3.4 us per wave,
 // then the second step's round trip).
-template <int R, int S> constexpr int npf_for() { return R * S >= 4 ? 1 : 4; }
-
 inline bool two_steps(int64_t m, int splitk) { return m / splitk <= 2048; }
 
-template <int G, int KIND, int S, int R, int SPLITK, int NPF, int NW = kWaves>
+template <int G, int KIND, int R, int SPLITK, int NPF, bool UA, int NW = kWaves>
 hipError_t launch_fast_t(const LinearArgs &a, const float *x, float *y, int64_t cap,
                          hipStream_t st) {
   const int64_t rows_per_group = SPLITK > 1 ? (int64_t)(NW / SPLITK) * R : (int64_t)NW * R;
@@ -460,32 +473,28 @@ hipError_t launch_fast_t(const LinearArgs &a, const float *x, float *y, int64_t 
   dim3 grid(grid_for(tiles, cap)), block(64 * NW);
   // x staged in LDS for rows up to the stage limit (and always in the
   // workgroups of K-split row groups), except when each lane's x slices fit
-  // in registers (one activation row, a wave K range of at most 2 steps):
-  // those are loaded before the weights and need no stage or barrier (the
-  // 8192 x 2048 linear: 6.40 -> 5.82 us)
-  const bool xreg = NW == kWaves && S == 1 && NPF <= 2 && a.m / SPLITK <= 1024 * NPF;
-  if ((NW > kWaves || S * a.m <= kLdsStageFloats) && !xreg) {
-    size_t lds = (size_t)S * a.m * sizeof(float);
-    hipLaunchKernelGGL((gemv_kernel<G, KIND, S, R, SPLITK, true, PRE_NONE, POST_STORE, NPF, NW>),
+  // in registers (a wave K range of at most 2 steps): those are loaded
+  // before the weights and need no stage or barrier (the 8192 x 2048
+  // linear: 6.40 -> 5.82 us)
+  const bool xreg = NW == kWaves && NPF <= 2 && a.m / SPLITK <= 1024 * NPF;
+  if ((NW > kWaves || a.m <= kLdsStageFloats) && !xreg) {
+    size_t lds = (size_t)a.m * sizeof(float);
+    hipLaunchKernelGGL((gemv_kernel<G, KIND, 1, R, SPLITK, true, PRE_NONE, POST_STORE, NPF, NW, UA>),
                        grid, block, lds, st, a.w, a.row_bytes, a.n, x, a.m, y, nullptr, 0.0f,
                        nullptr, nullptr);
   } else if constexpr (NW == kWaves) {
-    hipLaunchKernelGGL((gemv_kernel<G, KIND, S, R, SPLITK, false, PRE_NONE, POST_STORE, NPF>),
+    hipLaunchKernelGGL((gemv_kernel<G, KIND, 1, R, SPLITK, false, PRE_NONE, POST_STORE, NPF, NW, UA>),
                        grid, block, 0, st, a.w, a.row_bytes, a.n, x, a.m, y, nullptr, 0.0f,
                        nullptr, nullptr);
   }
   return hipGetLastError();
 }
 
-template <int G, int KIND, int S, int R, int SPLITK>
+template <int G, int KIND, int R, int SPLITK, bool UA>
 hipError_t launch_fast(const LinearArgs &a, const float *x, float *y, int64_t cap,
                        hipStream_t st) {
-  if constexpr (S == 1) {
-    if (two_steps(a.m, SPLITK)) return launch_fast_t<G, KIND, S, R, SPLITK, 2>(a, x, y, cap, st);
-    return launch_fast_t<G, KIND, S, R, SPLITK, 4>(a, x, y, cap, st);
-  } else {
-    return launch_fast_t<G, KIND, S, R, SPLITK, npf_for<R, S>()>(a, x, y, cap, st);
-  }
+  if (two_steps(a.m, SPLITK)) return launch_fast_t<G, KIND, R, SPLITK, 2, UA>(a, x, y, cap, st);
+  return launch_fast_t<G, KIND, R, SPLITK, 4, UA>(a, x, y, cap, st);
 }
 
 // Long rows at one activation row and at least 4096 outputs: the K split
@@ -501,47 +510,42 @@ hipError_t launch_fast(const LinearArgs &a, const float *x, float *y, int64_t ca
 // keep the 4-wave workgroups (with 8 waves the 1B down projection ran 6.0
 // against 5.9 us).  The stage holds m floats.
 inline bool long_row_groups(const LinearArgs &a) {
-  return a.s == 1 && a.m <= kLdsFloats && a.n >= 4096;
+  return a.m <= kLdsFloats && a.n >= 4096;
 }
 
 // Shape classes (tuned on MI355X, decode shapes of Llama-3.2-1B / Qwen3-8B):
 //   long rows (m > 4096):         K split over the 4 waves, 4 rows per workgroup
 //   vocabulary heads (n >= 64K):  2 rows per wave, up to 8192 workgroups
-//   one row, n >= 16384:          2 rows per wave, up to 2048 workgroups
+//   n >= 16384:                   2 rows per wave, up to 2048 workgroups
 //   wide (n >= 8192):             4 rows per wave, up to 1024 workgroups
-//   one row, n >= 4096:           2 rows per wave
+//   n >= 4096:                    2 rows per wave
 //   small:                        1 row per wave
-template <int G, int KIND, int S>
-hipError_t launch_rows(const LinearArgs &a, const float *x, float *y, hipStream_t st) {
+template <int G, int KIND, bool UA>
+hipError_t launch_rows(const LinearArgs &a, hipStream_t st) {
+  const float *x = reinterpret_cast<const float *>(a.x);
+  float *y = a.y;
   if (a.m > 4096 && a.m % 64 == 0) {
-    if constexpr (S == 1) {
-      if (long_row_groups(a)) return launch_fast_t<G, KIND, S, 4, 4, 2, 16>(a, x, y, 256, st);
-    }
-    return launch_fast<G, KIND, S, 4, 4>(a, x, y, 1024, st);
+    if (long_row_groups(a)) return launch_fast_t<G, KIND, 4, 4, 2, UA, 16>(a, x, y, 256, st);
+    return launch_fast<G, KIND, 4, 4, UA>(a, x, y, 1024, st);
   }
   // vocabulary heads: one K step in flight per wave (more waves per CU; the
   // 8192 workgroups walk about two row tiles each, so occupancy, not one
   // round of loads, covers the latency: 2 steps made the 1B lm_head 42 ->
   // 47 us)
-  if (a.n >= 65536) return launch_fast_t<G, KIND, S, 2, 1, 1>(a, x, y, 8192, st);
-  // one row, 16384 .. 65535 outputs: 2 rows per wave, up to 2048 workgroups
+  if (a.n >= 65536) return launch_fast_t<G, KIND, 2, 1, 1, UA>(a, x, y, 8192, st);
+  // 16384 .. 65535 outputs: 2 rows per wave, up to 2048 workgroups
   // (Qwen3-8B gate|up 4096 -> 24576: its decode-linears step 1.762 -> 1.750
   // ms; the 8192 x 2048 linear keeps 4 rows, 2 were 0.4-1.1 % slower)
-  if (S == 1 && a.n >= 16384) return launch_fast<G, KIND, S, 2, 1>(a, x, y, 2048, st);
-  if (a.n >= 8192) return launch_fast<G, KIND, S, 4, 1>(a, x, y, 1024, st);
-  // one row, 4096 .. 8191 outputs: 2 rows per wave (Qwen3-8B o and q|k|v)
-  if (S == 1 && a.n >= 4096) return launch_fast<G, KIND, S, 2, 1>(a, x, y, 2048, st);
-  return launch_fast<G, KIND, S, 1, 1>(a, x, y, 4096, st);
+  if (a.n >= 16384) return launch_fast<G, KIND, 2, 1, UA>(a, x, y, 2048, st);
+  if (a.n >= 8192) return launch_fast<G, KIND, 4, 1, UA>(a, x, y, 1024, st);
+  // 4096 .. 8191 outputs: 2 rows per wave (Qwen3-8B o and q|k|v)
+  if (a.n >= 4096) return launch_fast<G, KIND, 2, 1, UA>(a, x, y, 2048, st);
+  return launch_fast<G, KIND, 1, 1, UA>(a, x, y, 4096, st);
 }
 
 template <int G, int KIND>
 hipError_t launch_g(const LinearArgs &a, hipStream_t st) {
-  const float *x = reinterpret_cast<const float *>(a.x);
-  const bool aligned = !a.x_is_bf16 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0 &&
-                       a.row_bytes % 16 == 0 &&
-                       ((a.m / G) * ScaleTraits<KIND>::bytes) % 16 == 0 &&
-                       reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  if (!aligned) {
+  if (a.s > 1 || a.x_is_bf16) {
     const int64_t tasks = a.s * a.n;
     dim3 grid(grid_for((tasks + kWaves - 1) / kWaves, 4096)), block(256);
     if (a.x_is_bf16)
@@ -552,21 +556,11 @@ hipError_t launch_g(const LinearArgs &a, hipStream_t st) {
                          a.w, a.row_bytes, a.n, a.x, a.s, a.m, a.y);
     return hipGetLastError();
   }
-  // Batches of up to 4 activation rows per pass over the weights.
-  for (int64_t b0 = 0; b0 < a.s; b0 += 4) {
-    const int64_t sb = a.s - b0 < 4 ? a.s - b0 : 4;
-    const float *xb = x + b0 * a.m;
-    float *yb = a.y + b0 * a.n;
-    hipError_t e;
-    switch (sb) {
-      case 1: e = launch_rows<G, KIND, 1>(a, xb, yb, st); break;
-      case 2: e = launch_rows<G, KIND, 2>(a, xb, yb, st); break;
-      case 3: e = launch_rows<G, KIND, 3>(a, xb, yb, st); break;
-      default: e = launch_rows<G, KIND, 4>(a, xb, yb, st); break;
-    }
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  const bool aligned = reinterpret_cast<uintptr_t>(a.w) % 16 == 0 && a.row_bytes % 16 == 0 &&
+                       ((a.m / a.G) * ScaleTraits<KIND>::bytes) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(a.x) % 16 == 0;
+  if (aligned) return launch_rows<G, KIND, false>(a, st);
+  return launch_rows<G, KIND, true>(a, st);
 }
 
 template <int G, int KIND, int R, int SPLITK, int PRE, int POST, int NPF, int NW = kWaves>

@@ -97,6 +97,12 @@ hipError_t launch_skinny(const LinearArgs &a, hipStream_t st);
 constexpr int kSkinny4MaxRows = 4;
 hipError_t launch_skinny4(const LinearArgs &a, hipStream_t st);
 
+// Any alignment, f32 or bf16 x: binary16 fragments of x in `bytes` of scratch
+// (16-byte aligned), then MFMA on the codes as read; in chunks of as many rows as
+// mid_rows gives (0: a row tile does not fit, hipErrorInvalidValue).
+int64_t mid_rows(int64_t bytes, int64_t m, bool x_is_bf16);
+hipError_t launch_mid(const LinearArgs &a, void *scratch, int64_t bytes, hipStream_t st);
+
 struct GatherArgs {
   const uint8_t *w;      // byte address of packed row 0 of the table
   int64_t row_bytes;

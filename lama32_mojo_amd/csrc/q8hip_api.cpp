@@ -486,17 +486,25 @@ struct Scratch {
   int64_t act_bytes;
 };
 
-// The W8A32 linear of q8_linear on resolved pointers: GEMM from
-// kGemmMinRows rows, the few-row and small-batch MFMA kernels from
-// kSkinnyMinRows, the GEMV otherwise (and for unaligned operands).
+// Operands that are not 16-byte aligned, two rows and up or bf16 x: the
+// fragment MFMA path; the generic GEMV when a tile of 32 rows does not fit
+// the activation buffer (rows of 500 thousand values in 64 MiB).
+hipError_t run_unaligned(const q8::LinearArgs &la, void *act16, int64_t bytes, hipStream_t st) {
+  if (q8::mid_rows(bytes, la.m, la.x_is_bf16) > 0) return q8::launch_mid(la, act16, bytes, st);
+  return q8::launch_gemv(la, st);
+}
+
+// The W8A32 linear of q8_linear on resolved pointers: one row on the GEMV;
+// more on the GEMM from kGemmMinRows rows, below on the few-row and
+// small-batch MFMA kernels, and on the fragment MFMA path at any alignment.
 hipError_t dispatch_linear(q8::LinearArgs la, const Scratch &sc, hipStream_t st) {
   la.ws = sc.ws;
   la.ws_floats = sc.ws_floats;
-  if (la.s >= kGemmMinRows && gemm_aligned(la)) return run_gemm_in(la, sc.act16, sc.act_bytes, st);
-  if (la.s >= kSkinnyMinRows && la.s <= q8::kSkinny4MaxRows && gemm_aligned(la))
-    return q8::launch_skinny4(la, st);
-  if (la.s >= kSkinnyMinRows && gemm_aligned(la)) return q8::launch_skinny(la, st);
-  return q8::launch_gemv(la, st);
+  if (la.s < kSkinnyMinRows) return q8::launch_gemv(la, st);
+  if (!gemm_aligned(la)) return run_unaligned(la, sc.act16, sc.act_bytes, st);
+  if (la.s >= kGemmMinRows) return run_gemm_in(la, sc.act16, sc.act_bytes, st);
+  if (la.s <= q8::kSkinny4MaxRows) return q8::launch_skinny4(la, st);
+  return q8::launch_skinny(la, st);
 }
 
 Scratch ctx_scratch(q8_ctx *ctx) {
@@ -577,11 +585,11 @@ int q8_linear_bf16act(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *x, uint6
   la.G = G;
   la.kind = scale_dtype;
   hipError_t e;
-  if (gemm_aligned(la)) {
+  attach_gemm_workspace(ctx, la);
+  if (gemm_aligned(la))
     e = run_gemm(ctx, la);
-  } else {
-    e = q8::launch_gemv(la, ctx->stream);
-  }
+  else
+    e = run_unaligned(la, ctx->act16, kAct16Bytes, ctx->stream);
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_linear_bf16act launch");
   return ok(ctx);
 }

@@ -291,6 +291,90 @@ def test_linear_unaligned_weights(ctx, cor, G, scale):
     assert max_rel_err(y, cor.linear_f64(pk, x, G, scale)) <= TOL
 
 
+# (s, m, n): rows around the 32-row tiles, outputs around the 32-, 128- and
+# 256-column ones, K of one group, of a half unit of 32 codes, of a K split
+# (over waves at s = 1, over workgroups above), and a vocabulary-sized n
+UNALIGNED = [(1, 96, 7), (1, 1600, 333), (1, 4160, 4100), (1, 1600, 9000), (1, 672, 65600),
+             (2, 96, 1), (5, 1600, 31), (31, 544, 129), (32, 1600, 333), (33, 608, 257),
+             (65, 4160, 100), (200, 1600, 300), (430, 40032, 5)]
+
+
+@pytest.mark.parametrize("G,scale", LAYOUTS + [(32, "f16"), (64, "f32")])
+@pytest.mark.parametrize("s,m,n", UNALIGNED)
+@pytest.mark.parametrize("act", ["f32", "bf16"])
+def test_linear_any_alignment(ctx, cor, G, scale, s, m, n, act):
+    """Packed rows at an offset of 3 u16, whose lengths are mostly no
+    multiple of 16 bytes, and x one element off: one row on the GEMV,
+    more rows (and bf16 x) as binary16 fragments on the matrix cores, every
+    product exact in f32.  Bar: the f32 sums of a row, at most m / 32 group
+    partials of 32 products each, stay within (m / 32 + 32) 2^-24 of
+    float64 normwise (7.5e-5 at m = 40032); 1e-5 is asked below that."""
+    if m % G:
+        pytest.skip("rows hold whole groups")
+    say("any alignment", G, scale, s, m, n, act)
+    pk = cor.pack_bf16(synth_weights_bf16(n, m, seed=n + s), G, scale)
+    x = synth_x(s, m, seed=s + m)
+    if act == "bf16":
+        xbits = f32_to_bf16_bits(x)
+        w = upload(ctx, np.concatenate([np.zeros(3, np.uint16), pk.reshape(-1)]))
+        xb = upload(ctx, np.concatenate([np.zeros(1, np.uint16), xbits.reshape(-1)]))
+        yb = ctx.alloc(4 * s * n)
+        q8hip.linear_bf16act(ctx, w, 3, xb, 1, yb, 0, s, m, n, G, scale)
+        y = yb.download((s, n), np.float32)
+        for buf in (w, xb, yb):
+            buf.free()
+        x = bf16_bits_to_f32(xbits)
+    else:
+        y = gpu_linear(ctx, pk, x, G, scale, owt=3, pad_x=1)
+    ref = cor.linear_f64(pk, x, G, scale)
+    for b in range(s):
+        assert max_rel_err(y[b], ref[b]) <= 1e-5, b
+    assert elementwise_err(y, ref, cor.linear_abs(pk, x, G, scale)) <= 1e-5
+
+
+def test_linear_unaligned_infinities_and_tiny_rows(ctx, cor):
+    """An infinity or NaN in one activation row reaches only that row's
+    outputs (inf times a code keeps the code's sign, times 0 is NaN), and
+    rows from 1e-38 to 1e30 keep their precision (1e-5, as above)."""
+    say("unaligned inf / NaN")
+    G, scale, s, m, n = 32, "f32", 40, 1632, 65
+    pk = cor.pack_bf16(synth_weights_bf16(n, m, seed=3), G, scale)
+    x = synth_x(s, m, seed=4)
+    for i, f in enumerate([1e-38, 1e-30, 1e-10, 1e10, 1e30]):
+        x[10 + i] *= f / np.abs(x[10 + i]).max()
+    x[20] = 0.0
+    ref = cor.linear_f64(pk, x, G, scale)
+    x[1, 5] = np.inf
+    x[33, 700] = -np.inf
+    x[2, 7] = np.nan
+    y = gpu_linear(ctx, pk, x, G, scale, owt=1)
+    codes, _ = unpack_q8_np(pk, m, G, scale)
+    for b in set(range(s)) - {1, 2, 20, 33}:
+        assert max_rel_err(y[b], ref[b]) <= 1e-5, b
+    assert np.all(y[20] == 0.0) and np.all(np.isnan(y[2]))
+    for b, k, sign in ((1, 5, 1.0), (33, 700, -1.0)):
+        q = codes[:, k].astype(np.float32)
+        with np.errstate(invalid="ignore"):
+            want = sign * np.float32(np.inf) * q
+        assert np.array_equal(y[b], want, equal_nan=True), b
+
+
+def test_linear_unaligned_rows_past_the_scratch(cor):
+    """Rows whose 32-row fragment tile does not fit the allocation-free
+    scratch (131104 codes: 16.8 MB) run on the generic GEMV."""
+    import torch
+    say("unaligned, past the scratch")
+    G, scale, s, m, n = 32, "f16", 2, 131104, 3
+    pk = cor.pack_bf16(synth_weights_bf16(n, m, seed=5), G, scale)
+    x = synth_x(s, m, seed=6)
+    w = torch.from_numpy(pk.view(np.int16)).cuda()
+    xt, y = torch.from_numpy(x).cuda(), torch.zeros((s, n), device="cuda")
+    torch.cuda.synchronize()
+    q8hip.linear_noalloc(None, w.data_ptr(), xt.data_ptr(), y.data_ptr(), s, m, n, G, scale)
+    torch.cuda.synchronize()
+    assert max_rel_err(y.cpu().numpy(), cor.linear_f64(pk, x, G, scale)) <= 2e-5
+
+
 def test_linear_lm_head_full_size(ctx, cor):
     """Llama-3.2-1B tied lm_head, 128256 x 2048, s = 1."""
     say("lm_head full size")
