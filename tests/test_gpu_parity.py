@@ -92,6 +92,24 @@ def test_pack_matches_oracle_llama_up_proj(ctx, cor, G, scale, src):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("G,scale", LAYOUTS + [(32, "f16"), (64, "f32")])
+def test_pack_near_ties(ctx, cor, G, scale):
+    """Weights within a few f32 ulps of (k + 1/2) * scale, on both sides and
+    on the tie: the codes are those of the correctly rounded quotient, bit
+    for bit."""
+    say("pack near ties", G, scale)
+    rng = np.random.default_rng(11)
+    n, m = 256, 2048
+    s = np.exp2(rng.integers(-12, 4, (n, m // G))) * (1.0 + rng.integers(0, 1024, (n, m // G)) / 1024)
+    k = rng.integers(-127, 127, (n, m // G, G)) + 0.5
+    w = (k * s[:, :, None]).astype(np.float32)
+    w = (w.view(np.int32) + rng.integers(-6, 7, w.shape, dtype=np.int32)).view(np.float32)
+    w[:, :, 0] = 127.0 * s
+    w = np.ascontiguousarray(w.reshape(n, m))
+    got = q8.pack_q8_bits(w, G, scale, ctx, src_dtype="f32")
+    assert np.array_equal(got, cor.pack_f32(w, G, scale))
+
+
 def test_pack_f32_wide_dynamic_range(ctx, cor):
     """f32 inputs that are not bf16 values, spanning many binades."""
     say("pack f32 wide range")
