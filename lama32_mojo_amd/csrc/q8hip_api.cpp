@@ -424,6 +424,14 @@ bool gemm_aligned(const q8::LinearArgs &a) {
 // on f16 MFMA.
 constexpr int64_t kSkinnyMinRows = 2;
 constexpr int64_t kGemmMinRows = 32;
+// 17 .. 31 rows of at least this many codes take the fragment MFMA path,
+// which reads each code once per 32 rows; on shorter rows its two extra
+// launches cost more than that saves (17 and 31 rows, small-batch kernel ->
+// fragments: 4096 x 6144 23.1 / 32.7 -> 17.4 / 18.2 us, 4096 x 24576 55.0 /
+// 64.6 -> 43.3 / 44.0, 12288 x 4096 33.2 -> 23.8 at 17, 8192 x 2048 22.9 /
+// 32.3 -> 16.2 / 17.9; but 2048 x 16384 16.4 / 21.0 -> 17.4 / 18.2, 1024 x
+// 6144 7.8 / 10.3 -> 11.0 / 12.0).
+constexpr int64_t kMidMinWidth = 4096;
 
 // Attach the context's split-K workspace to a launch.
 void attach_gemm_workspace(q8_ctx *ctx, q8::LinearArgs &la) {
@@ -504,6 +512,8 @@ hipError_t dispatch_linear(q8::LinearArgs la, const Scratch &sc, hipStream_t st)
   if (!gemm_aligned(la)) return run_unaligned(la, sc.act16, sc.act_bytes, st);
   if (la.s >= kGemmMinRows) return run_gemm_in(la, sc.act16, sc.act_bytes, st);
   if (la.s <= q8::kSkinny4MaxRows) return q8::launch_skinny4(la, st);
+  if (la.s > 16 && la.m >= kMidMinWidth && q8::mid_rows(sc.act_bytes, la.m, 0) > 0)
+    return q8::launch_mid(la, sc.act16, sc.act_bytes, st);
   return q8::launch_skinny(la, st);
 }
 

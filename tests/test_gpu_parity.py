@@ -350,6 +350,21 @@ def test_linear_any_alignment(ctx, cor, G, scale, s, m, n, act):
     assert elementwise_err(y, ref, cor.linear_abs(pk, x, G, scale)) <= 1e-5
 
 
+@pytest.mark.parametrize("G,scale", LAYOUTS)
+@pytest.mark.parametrize("s,m,n", [(17, 4096, 33), (31, 4096, 4100), (23, 12288, 1), (16, 4096, 33),
+                                   (31, 3584, 130)])
+def test_linear_17_to_31_rows(ctx, cor, G, scale, s, m, n):
+    """17 .. 31 aligned rows of 4096 codes and more take the fragment path,
+    16 rows and shorter ones the small-batch kernel: both within 1e-5."""
+    say("17 to 31 rows", G, scale, s, m, n)
+    pk = cor.pack_bf16(synth_weights_bf16(n, m, seed=n + s), G, scale)
+    x = synth_x(s, m, seed=s + m)
+    y = gpu_linear(ctx, pk, x, G, scale)
+    ref = cor.linear_f64(pk, x, G, scale)
+    for b in range(s):
+        assert max_rel_err(y[b], ref[b]) <= 1e-5, b
+
+
 def test_linear_unaligned_infinities_and_tiny_rows(ctx, cor):
     """An infinity or NaN in one activation row reaches only that row's
     outputs (inf times a code keeps the code's sign, times 0 is NaN), and
