@@ -303,7 +303,7 @@ int q8_rope_kv(q8_ctx *ctx, q8_buf *a, uint64_t oq_f32, uint64_t ok_f32,
                int head_dim, int64_t ld);
 
 /* Floats of activation-arena scratch q8_attention needs (0 from s = 16 on,
- * where attention is one pass on the matrix cores). */
+ * where attention always runs on the matrix cores). */
 uint64_t q8_attention_scratch_floats(int64_t s, int nheads, int head_dim,
                                      int64_t maxlen);
 
@@ -312,9 +312,12 @@ uint64_t q8_attention_scratch_floats(int64_t s, int nheads, int head_dim,
  * 0 .. pos0 + i; head h reads KV head h / (nheads / nkv); scores scaled by
  * 1/sqrt(head_dim)) -- k_scores, k_softmax_rows and k_att_out
  * (src/llama_common.mojo:402-473) with their score buffer replaced by an
- * online softmax: for s >= 16 one MFMA pass per (16..128-row block, KV
- * head), below that per-split partials in q8_attention_scratch_floats()
- * floats at oscratch (oscratch is unused when that is 0).  head_dim 64 or
+ * online softmax: one MFMA pass per (16..128-row block, KV head), whose keys
+ * are split over several blocks where few rows meet a long cache (the split
+ * records live in the context's workspace, so calls on one context must not
+ * overlap).  Below 16 rows operands that are not 16-byte aligned take
+ * per-split partials in q8_attention_scratch_floats() floats at oscratch
+ * (oscratch is unused when that is 0).  head_dim 64 or
  * 128, nheads / nkv in {1, 2, 4, 8}.  Position as in q8_rope_kv.  Row i of q
  * at oq + i*ldq (ldq = 0: nheads*head_dim, dense); out is dense.  From
  * s = 16 on, q and out must start 16-byte aligned and ldq be a multiple of 4

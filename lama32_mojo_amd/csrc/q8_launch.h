@@ -138,6 +138,10 @@ struct AttnArgs {
   int pos0;
   int maxlen;            // cache rows; positions past it are clamped
   int64_t ldq;           // q row stride in floats (nheads * head_dim when dense)
+  // scratch of the MFMA pass's key splits (null: no split)
+  float *ws = nullptr;
+  int64_t ws_floats = 0;
+  bool mfma_ok = false;  // fewer rows may take the MFMA pass (16-byte aligned q, out, rows)
 };
 // Row counts from which attention runs as one MFMA pass per (row block, KV
 // head) with no scratch; below it, as (KV head, 64-key split) partials

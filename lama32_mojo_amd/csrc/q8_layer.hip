@@ -261,12 +261,31 @@ __device__ __forceinline__ void split_f16(float a, _Float16 &hi, _Float16 &lo) {
 // the accumulators stay in VGPRs (no AGPR copies around the rescale) and one
 // block's MFMAs run beside the other's softmax (2048 rows, 128-dim heads
 // 32 / 8: 126 -> 113 us; one block per CU took 328 registers).
-template <int HD, int GRP>
+//
+// SPLIT: a grid with few row blocks also splits the keys, gridDim.z blocks
+// per (KV head, row block), each over an equal run of the row block's key
+// tiles (split_tiles); a block writes its unnormalised output rows, running
+// maximum and sum to part ([z][row][head][HD], behind it [z][row][head][2])
+// for attn_prefill_merge_kernel.  A row block whose tiles are not split is
+// served by its block 0, which writes the output (the bits of the unsplit
+// kernel).  Before this, 16 rows after 4000 cached ones ran on 8 blocks:
+// 152 -> 20 us (32 / 8 heads of 128), 256 rows 163 -> 69 us; 15 rows, which
+// took one pass per row, 122 -> 20 us.
+// Key tiles per block when nz blocks share ntiles: all of them unless
+// sharing shortens the longest chain by 6 tiles, about what the merge launch
+// costs (0.8-1.2 us a tile; 512 rows of 64-dim heads 18.2 us whole, 19.5 in
+// two; 700 rows of 128-dim heads, 11 tiles, 32.7 and 30.5).
+__host__ __device__ inline int split_tiles(int ntiles, int nz) {
+  const int t = (ntiles + nz - 1) / nz;
+  return ntiles - t >= 6 ? t : ntiles;
+}
+template <int HD, int GRP, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_prefill_kernel(const float *__restrict__ q,
                                                            const __half *__restrict__ kc,
                                                            const __half *__restrict__ vc,
-                                                           float *__restrict__ out, int s,
+                                                           float *__restrict__ out,
+                                                           float *__restrict__ part, int s,
                                                            int nheads, int nkv, const int *posp,
                                                            int pos0_host, int maxlen,
                                                            int64_t ldq) {
@@ -291,7 +310,15 @@ void attn_prefill_kernel(const float *__restrict__ q,
   const int row0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * PB;   // longest rows first
   const int nkeys = min(pos0 + min(row0 + PB, s), maxlen);   // keys any row of the block sees
   const int ntiles = nkeys > 0 ? (nkeys + BK - 1) / BK : 0;
-  const int wend = min(pos0 + min(row0 + w * PW + PW, s), maxlen);   // ... any row of the wave
+  // this block's tiles; with one run for all (apart == false) only block 0
+  // has any
+  const int tps = SPLIT ? split_tiles(ntiles, (int)gridDim.z) : ntiles;
+  const bool apart = SPLIT && tps < ntiles;
+  const int kt0 = SPLIT ? (int)blockIdx.z * tps : 0;
+  const int kt1 = SPLIT ? min(kt0 + tps, ntiles) : ntiles;
+  if (SPLIT && kt0 >= ntiles && blockIdx.z > 0) return;
+  // ... any row of the wave (none: a wave past the rows)
+  const int wend = row0 + w * PW < s ? min(pos0 + min(row0 + w * PW + PW, s), maxlen) : 0;
   const int wfull = min(pos0 + min(row0 + w * PW, s - 1) + 1, maxlen);  // ... every row of it
   const int i = row0 + w * PW + col / GRP;       // this lane's column: row i, head
   const int head = g * GRP + col % GRP;
@@ -383,12 +410,12 @@ void attn_prefill_kernel(const float *__restrict__ q,
 #pragma unroll
     for (int v = 0; v < 16; ++v) o[t][v] = 0.0f;
   float m = -INFINITY, l = 0.0f;
-  if (ntiles > 0) load_tile(0);
-  for (int kt = 0; kt < ntiles; ++kt) {
+  if (kt0 < kt1) load_tile(kt0);
+  for (int kt = kt0; kt < kt1; ++kt) {
     __syncthreads();                             // every wave is done with the last tile
     store_tile();
     __syncthreads();
-    if (kt + 1 < ntiles) load_tile(kt + 1);
+    if (kt + 1 < kt1) load_tile(kt + 1);
     const int k0 = kt * BK;
     if (k0 >= wend) continue;                    // past every row of this wave
     f32x16 sc[2];
@@ -406,7 +433,7 @@ void attn_prefill_kernel(const float *__restrict__ q,
     // online softmax of the column over this tile (the other 32 keys of the
     // tile live in lane l ^ 32); a tile every row of the wave sees whole
     // needs no causal mask
-    float tmax = -INFINITY;
+    float tmax = -INFINITY, m_new;
     if (k0 + BK <= wfull) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -428,9 +455,12 @@ void attn_prefill_kernel(const float *__restrict__ q,
         }
     }
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-    const float mn = fmaxf(m, tmax);             // finite: key 0 is visible to every column
+    // finite without a split: key 0 is visible to every column; a split's
+    // tiles may all lie past a column's row (then every p and alpha is 0)
+    m_new = fmaxf(m, tmax);
+    const float mn = SPLIT && m_new == -INFINITY ? 0.0f : m_new;
     const float alpha = exp2f(m - mn);
-    m = mn;
+    m = m_new;
     float ps = 0.0f;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -472,8 +502,9 @@ void attn_prefill_kernel(const float *__restrict__ q,
   }
   l += __shfl_xor(l, 32);
   if (i < s) {
-    const float il = 1.0f / (l * 16384.0f);
-    float *orow = out + (int64_t)i * qdim + head * HD + 4 * hf;
+    const float il = apart ? 1.0f / 16384.0f : 1.0f / (l * 16384.0f);
+    const int64_t rec = (int64_t)blockIdx.z * s + i;
+    float *orow = (apart ? part + rec * qdim : out + (int64_t)i * qdim) + head * HD + 4 * hf;
 #pragma unroll
     for (int d = 0; d < DT; ++d)
 #pragma unroll
@@ -483,7 +514,66 @@ void attn_prefill_kernel(const float *__restrict__ q,
         for (int c = 0; c < 4; ++c) r[c] = o[d][4 * vb + c] * il;
         *reinterpret_cast<f32x4 *>(orow + 32 * d + 8 * vb) = r;
       }
+    if (apart && hf == 0) {
+      float2 *ml = reinterpret_cast<float2 *>(part + (int64_t)gridDim.z * s * qdim);
+      ml[rec * nheads + head] = make_float2(m, l);
+    }
   }
+}
+
+// out = sum_z f_z o_z / sum_z f_z l_z, f_z = 2^(m_z - max m), over the
+// splits of a (row, head) that hold tiles; one thread per 4 dims, the loads
+// of 8 splits at a time issued together.  Rows served whole are left alone.
+template <int HD, int GRP>
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float *__restrict__ part,
+                                                                 float *__restrict__ out, int s,
+                                                                 int nheads, int nz,
+                                                                 const int *posp, int pos0_host,
+                                                                 int maxlen) {
+  constexpr int PB = 4 * (32 / GRP);                 // as attn_prefill_kernel
+  const int64_t rows = (int64_t)s * nheads;          // (row, head) records
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t r = t / (HD / 4);
+  if (r >= rows) return;
+  const int pos0 = posp ? *posp : pos0_host;
+  const int row0 = (int)(r / nheads) / PB * PB;
+  const int nkeys = min(pos0 + min(row0 + PB, s), maxlen);
+  const int ntiles = nkeys > 0 ? (nkeys + kPrefillBK - 1) / kPrefillBK : 0;
+  const int tps = split_tiles(ntiles, nz);
+  if (tps >= ntiles) return;
+  const int64_t nz_all = nz;
+  nz = (ntiles + tps - 1) / tps;                     // splits with tiles
+  const float2 *ml = reinterpret_cast<const float2 *>(part + nz_all * rows * HD);
+  const int d = 4 * (int)(t % (HD / 4));
+  float m = -INFINITY, l = 0.0f;
+  f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int z0 = 0; z0 < nz; z0 += 8) {
+    float2 a[8];
+    f32x4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int z = z0 + u < nz ? z0 + u : nz - 1;
+      a[u] = ml[z * rows + r];
+      v[u] = *reinterpret_cast<const f32x4 *>(part + (z * rows + r) * HD + d);
+    }
+    // (split 0 holds key 0, which every row sees: the maximum is finite)
+    float mx = m;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) mx = fmaxf(mx, z0 + u < nz ? a[u].x : -INFINITY);
+    const float f0 = exp2f(m - mx);
+    l *= f0;
+    o *= f0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float f = z0 + u < nz ? exp2f(a[u].x - mx) : 0.0f;
+      l = __builtin_fmaf(f, a[u].y, l);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c] = __builtin_fmaf(f, v[u][c], o[c]);
+    }
+    m = mx;
+  }
+  const float il = 1.0f / l;
+  *reinterpret_cast<f32x4 *>(out + r * HD + d) = f32x4{o.x * il, o.y * il, o.z * il, o.w * il};
 }
 
 // ---- decode attention: RoPE + KV append + attention of one new token --------
@@ -982,18 +1072,41 @@ hipError_t launch_attn_t(const AttnArgs &a, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Key splits of the prompt-row kernel: about one block per CU in all, within
+// the scratch (512 blocks: 15 rows after 4000 20 -> 27 us).  They are
+// counted for the whole cache, so a device position gives the splits, and
+// with them the bits, of a host position.
 template <int HD, int GRP>
 hipError_t launch_prefill_t(const AttnArgs &a, hipStream_t st) {
   constexpr int PB = 4 * (32 / GRP);
-  hipLaunchKernelGGL((attn_prefill_kernel<HD, GRP>), dim3((unsigned)a.nkv, (unsigned)((a.s + PB - 1) / PB)),
-                     dim3(256), 0, st, a.q, a.kc, a.vc, a.out, a.s, a.nheads, a.nkv, a.posp,
-                     a.pos0, a.maxlen, a.ldq);
+  const int64_t rb = (a.s + PB - 1) / PB;
+  const int64_t rec = (int64_t)a.s * a.nheads * (HD + 2);
+  int64_t nz = 256 / (a.nkv * rb);
+  const int64_t tiles = ((int64_t)a.maxlen + kPrefillBK - 1) / kPrefillBK;
+  nz = nz < tiles ? nz : tiles;
+  nz = nz < a.ws_floats / rec ? nz : a.ws_floats / rec;
+  // With the position known here: nothing to split, no merge launch.
+  const int64_t keys = a.posp || a.pos0 + (int64_t)a.s > a.maxlen ? a.maxlen : a.pos0 + a.s;
+  const int most = (int)((keys + kPrefillBK - 1) / kPrefillBK);
+  if (nz <= 1 || !a.ws || split_tiles(most, (int)nz) >= most) {
+    hipLaunchKernelGGL((attn_prefill_kernel<HD, GRP, false>), dim3((unsigned)a.nkv, (unsigned)rb),
+                       dim3(256), 0, st, a.q, a.kc, a.vc, a.out, nullptr, a.s, a.nheads, a.nkv,
+                       a.posp, a.pos0, a.maxlen, a.ldq);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((attn_prefill_kernel<HD, GRP, true>),
+                     dim3((unsigned)a.nkv, (unsigned)rb, (unsigned)nz), dim3(256), 0, st, a.q, a.kc,
+                     a.vc, a.out, a.ws, a.s, a.nheads, a.nkv, a.posp, a.pos0, a.maxlen, a.ldq);
+  const int64_t threads = (int64_t)a.s * a.nheads * (HD / 4);
+  hipLaunchKernelGGL((attn_prefill_merge_kernel<HD, GRP>), dim3(blocks_for(threads, 256)),
+                     dim3(256), 0, st, a.ws, a.out, a.s, a.nheads, (int)nz, a.posp, a.pos0,
+                     a.maxlen);
   return hipGetLastError();
 }
 
 template <int HD>
 hipError_t launch_attn_hd(const AttnArgs &a, hipStream_t st) {
-  const bool mfma = a.s >= kPrefillMinRows;
+  const bool mfma = a.s >= kPrefillMinRows || a.mfma_ok;
   switch (a.nheads / a.nkv) {
     case 1: return mfma ? launch_prefill_t<HD, 1>(a, st) : launch_attn_t<HD, 1>(a, st);
     case 2: return mfma ? launch_prefill_t<HD, 2>(a, st) : launch_attn_t<HD, 2>(a, st);

@@ -1292,6 +1292,14 @@ int q8_attention(q8_ctx *ctx, q8_buf *a, uint64_t oq_f32, q8_buf *kv, uint64_t o
   aa.pos0 = (int)pos0;
   aa.maxlen = (int)maxlen;
   aa.ldq = ldq;
+  aa.ws = ctx->gemm_ws;
+  aa.ws_floats = kGemmWsFloats;
+  // fewer rows than kPrefillMinRows take the MFMA pass too where their
+  // operands are aligned for it
+  aa.mfma_ok = reinterpret_cast<uintptr_t>(aa.q) % 16 == 0 &&
+               reinterpret_cast<uintptr_t>(aa.out) % 16 == 0 && ldq % 4 == 0 &&
+               reinterpret_cast<uintptr_t>(aa.kc) % 16 == 0 &&
+               reinterpret_cast<uintptr_t>(aa.vc) % 16 == 0;
   hipError_t e = q8::launch_attention(aa, ctx->stream);
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_attention launch");
   return ok(ctx);

@@ -159,6 +159,50 @@ def test_attention(ctx, head_dim, nh, nkv, s, pos0):
         b.free()
 
 
+@pytest.mark.parametrize("head_dim,nh,nkv", [(128, 8, 2), (64, 16, 2), (128, 4, 4), (64, 4, 2)])
+@pytest.mark.parametrize("s,pos0,maxlen", [(2, 3000, 3002), (15, 447, 2048), (16, 448, 2048),
+                                           (33, 1000, 4096), (700, 0, 700), (40, 0, 4096),
+                                           (129, 2900, 3029)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_attention_key_splits(ctx, head_dim, nh, nkv, s, pos0, maxlen, shift):
+    """Few rows over a long cache split the keys over blocks: up to one split
+    per 64-key tile, rows that see none of a later split's keys (700 rows
+    from position 0), caches mostly past the context (served whole), and 2 to
+    15 rows, which with shift = 1 (q one float off 16 bytes) keep the
+    per-row kernels.  Within 1e-5 of float64 row by row, a NaN past the
+    context reaches nothing, and a device position gives the same bits."""
+    if shift and s >= 16:
+        pytest.skip("16 rows and up must be aligned")
+    say("attention splits", head_dim, nh, nkv, s, pos0, maxlen, shift)
+    rng = np.random.default_rng(s + pos0)
+    qd, kvd = nh * head_dim, nkv * head_dim
+    cache = np.full((2, maxlen, kvd), np.nan, np.float16)
+    cache[0, :pos0 + s] = rng.standard_normal((pos0 + s, kvd)) * 0.7
+    cache[1, :pos0 + s] = rng.standard_normal((pos0 + s, kvd))
+    q = rng.standard_normal((s, qd)).astype(np.float32)
+    kv = ctx.alloc(cache.nbytes)
+    kv.upload(cache)
+    scr = q8hip.attention_scratch_floats(s, nh, head_dim, maxlen)
+    oq, oy, osc = shift, shift + s * qd, shift + 2 * s * qd
+    a = arena(ctx, osc + scr)
+    put(a, oq, q)
+    pb = ctx.alloc(16)
+    pb.upload(np.array([0, pos0, 0, 0], np.int32))
+    out = []
+    for host in (True, False):
+        put(a, oy, np.zeros((s, qd), np.float32))
+        q8hip.attention(ctx, a, oq, kv, 0, maxlen * kvd, maxlen, oy, osc, s, pos0 if host else 0,
+                        nh, nkv, head_dim, posbuf=None if host else pb, opos_i32=1)
+        out.append(get(a, oy, (s, qd)))
+    assert np.array_equal(out[0], out[1])
+    c = cache[:, :pos0 + s].astype(np.float64)
+    ref = mo.attention(q.astype(np.float64), c[0], c[1], pos0, nh, nkv, head_dim)
+    for i in range(s):
+        assert max_rel_err(out[0][i], ref[i]) <= 1e-5, i
+    for b in (a, kv, pb):
+        b.free()
+
+
 @pytest.mark.parametrize("head_dim,nh,nkv,s", [(64, 8, 2, 3), (128, 32, 8, 48),
                                                (64, 32, 8, 130)])
 def test_stacked_qkv_rows_equal_dense(ctx, head_dim, nh, nkv, s):
