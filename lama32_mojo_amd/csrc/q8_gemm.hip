@@ -430,6 +430,9 @@ void gemm_kernel(const uint8_t *__restrict__ w, int64_t row_bytes,
         else
           S.sc[u] = __builtin_amdgcn_raw_buffer_load_b32(wr, o, 0, 0);
       }
+      // keep the loads of the iterations in this order: the waits below count
+      // the loads issued since
+      __builtin_amdgcn_sched_barrier(0);
     };
     auto store = [&](const Stage &S, int it, int buf) {
 #pragma unroll
@@ -461,17 +464,22 @@ void gemm_kernel(const uint8_t *__restrict__ w, int64_t row_bytes,
     __syncthreads();
     // iteration it: the consumers read LDS stage it & 1; write stage
     // (it + 1) & 1 (read last in iteration it - 1) from registers, which then
-    // load iteration it + 1 + PD
-    for (int it0 = 0; it0 < nit; it0 += PD) {
+    // load iteration it + 1 + PD.  nit is a multiple of PD and nothing here
+    // is conditional (what is stored or loaded past the last iteration is
+    // not used): a branch or an early exit made the compiler wait for every
+    // load in flight at the head of the loop, one iteration of prefetch
+    // instead of two (64 x 6144 x 4096 17.8 -> 16.2 us, 128 x 6144 x 4096
+    // 22.0 -> 19.1; four stages are no faster).
+    int it = 0;
+    do {
 #pragma unroll
       for (int u = 0; u < PD; ++u) {
-        const int it = it0 + u;
-        if (it >= nit) break;
-        if (it + 1 < nit) store(S[(u + 1) % PD], it + 1, (it + 1) & 1);
+        store(S[(u + 1) % PD], it + 1, (it + 1) & 1);
         load(S[(u + 1) % PD], it + 1 + PD);
         __syncthreads();
+        ++it;
       }
-    }
+    } while (it < nit);
     return;
   }
 
@@ -584,6 +592,17 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
   }
 }
 
+// Split K when the output tiles alone leave CUs idle (256 CUs, one workgroup
+// each); every split keeps at least 512 codes.
+int64_t k_splits(const LinearArgs &a, int64_t tiles) {
+  int64_t splits = 1;
+  if (a.ws)
+    while (tiles * splits * 2 <= 256 && (a.m + 2 * splits - 1) / (2 * splits) >= 512 &&
+           2 * splits * a.s * a.n <= a.ws_floats)
+      splits *= 2;
+  return splits;
+}
+
 template <int G, int KIND, int TM, int TN, int CR = 1, int NPW = kProducerWaves,
           int KS = kIterCodes>
 hipError_t launch_t(const LinearArgs &a, const uint16_t *x16, const int *ex, const int *ew,
@@ -591,15 +610,9 @@ hipError_t launch_t(const LinearArgs &a, const uint16_t *x16, const int *ex, con
   constexpr int BM = 32 * TM * CR, BN = 32 * TN * (4 / CR);
   const int64_t nit_all = (a.m + KS - 1) / KS;
   const int64_t gx = (a.n + BN - 1) / BN, gy = (a.s + BM - 1) / BM;
-  // Split K when the output tiles alone leave CUs idle (256 CUs, one
-  // workgroup each); every split keeps at least 512 codes.
-  int64_t splits = 1;
-  if (a.ws) {
-    while (gx * gy * splits * 2 <= 256 && (nit_all + 2 * splits - 1) / (2 * splits) >= 512 / KS &&
-           2 * splits * a.s * a.n <= a.ws_floats)
-      splits *= 2;
-  }
-  int64_t nit = (nit_all + splits - 1) / splits;
+  int64_t splits = k_splits(a, gx * gy);
+  const int64_t nit = ((nit_all + splits - 1) / splits + kStages - 1) / kStages * kStages;
+  splits = (nit_all + nit - 1) / nit;                  // no empty split
   dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)splits), block(64 * (4 + NPW));
   hipLaunchKernelGGL((gemm_kernel<G, KIND, TM, TN, CR, NPW, kStages, KS>), grid, block, 0, st, a.w, a.row_bytes,
                      x16, ex, ew, a.y, a.s, a.m, a.n, (int)nit, a.ws);
@@ -648,9 +661,19 @@ hipError_t launch_g(const LinearArgs &a, uint16_t *x16, int *ex, int *ew, bool w
       if ((a.n + 127) / 128 * rb64 <= 256)
         return launch_t<G, KIND, 2, 1, 1, kProducerWaves, 128>(a, x16, ex, ew, st);
     }
+    // 128 x 128 tiles take 128 codes per iteration too where a split has
+    // 4096 or more (128 x 28672 x 4096 56.5 -> 52.8 us, 512 x 4096 x 14336
+    // 101 -> 95.5; shorter ones lose: 512 x 2048 x 8192 in 4 splits 37.7 ->
+    // 39.0, 1024 x 6144 x 1024 31.1 -> 32.4).
+    const int64_t tiles = (a.n + 127) / 128 * ((a.s + 127) / 128);
+    if (a.m / k_splits(a, tiles) >= 4096)
+      return launch_t<G, KIND, 4, 1, 1, kProducerWaves, 128>(a, x16, ex, ew, st);
     return launch_t<G, KIND, 4, 1>(a, x16, ex, ew, st);
   }
-  return launch_t<G, KIND, 2, 1>(a, x16, ex, ew, st);
+  // up to 64 rows: 64 x 128 tiles, 128 codes per iteration (32 / 64 x 28672 x
+  // 4096 50.8 / 53.4 -> 38.5 / 41.1 us with the producers' two iterations of
+  // prefetch; equal on 6144 and 4096 outputs)
+  return launch_t<G, KIND, 2, 1, 1, kProducerWaves, 128>(a, x16, ex, ew, st);
 }
 
 }  // namespace

@@ -350,6 +350,28 @@ def test_linear_any_alignment(ctx, cor, G, scale, s, m, n, act):
     assert elementwise_err(y, ref, cor.linear_abs(pk, x, G, scale)) <= 1e-5
 
 
+@pytest.mark.parametrize("G,scale,s,m,n", [
+    (32, "f32", 33, 128, 64), (32, "f32", 64, 384, 127), (32, "f32", 65, 640, 129),
+    (32, "f32", 129, 1152, 128), (32, "f32", 257, 896, 8200), (32, "f32", 40, 4736, 24),
+    (32, "f16", 100, 4864, 500), (64, "f16", 128, 4608, 2049), (64, "f32", 130, 4352, 16500),
+    (64, "f16", 512, 8704, 1000), (64, "f16", 600, 1536, 24700)])
+def test_gemm_iteration_counts_and_ragged_tiles(ctx, cor, G, scale, s, m, n):
+    """Odd and even numbers of 64- and 128-code iterations (the last one of an
+    odd count runs on zeros), K splits that they do not divide, on every tile
+    shape, with whole and ragged tiles side by side.  Binary16 x (2^-12) and
+    weights (2^-11 or 2^-10): 5e-4 normwise, 1e-3 per row and of each
+    output's own scale."""
+    say("gemm iterations", G, scale, s, m, n)
+    pk = cor.pack_bf16(synth_weights_bf16(n, m, seed=n + s), G, scale)
+    x = synth_x(s, m, seed=s + m)
+    y = gpu_linear(ctx, pk, x, G, scale)
+    ref = cor.linear_f64(pk, x, G, scale)
+    for b in range(s):
+        assert max_rel_err(y[b], ref[b]) <= 1e-3, b
+    assert np.linalg.norm(y - ref) <= 5e-4 * np.linalg.norm(ref)
+    assert elementwise_err(y, ref, cor.linear_abs(pk, x, G, scale)) <= 1e-3
+
+
 @pytest.mark.parametrize("G,scale", LAYOUTS)
 @pytest.mark.parametrize("s,m,n", [(17, 4096, 33), (31, 4096, 4100), (23, 12288, 1), (16, 4096, 33),
                                    (31, 3584, 130)])
