@@ -499,22 +499,55 @@ void gemm_kernel(const uint8_t *__restrict__ w, int64_t row_bytes,
   for (int it = 0; it < nit; ++it) {
     const _Float16 *at = As[it & 1];
     const _Float16 *bt = Bs[it & 1];
-#pragma unroll
-    for (int ks = 0; ks < KS / 16; ++ks) {
-      // v_mfma_f32_32x32x16_f16 operands: lane (lr, lh) holds row / column lr,
-      // k = 16 ks + 8 lh .. +8 of this tile, for both A and B
-      f16x8 af[TM], bf[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        af[i] = *reinterpret_cast<const f16x8 *>(&at[(rb + i * 32 + lr) * LDS_ROW + 16 * ks + 8 * lh]);
+    // v_mfma_f32_32x32x16_f16 operands: lane (lr, lh) holds row / column lr,
+    // k = 16 ks + 8 lh .. +8 of this tile, for both A and B
+    auto read_a = [&](f16x8 &f, int ks, int i) {
+      f = *reinterpret_cast<const f16x8 *>(&at[(rb + i * 32 + lr) * LDS_ROW + 16 * ks + 8 * lh]);
+    };
+    auto read_b = [&](f16x8 (&f)[TN], int ks) {
 #pragma unroll
       for (int t = 0; t < TN; ++t)
-        bf[t] = *reinterpret_cast<const f16x8 *>(&bt[(cb + t * 32 + lr) * LDS_ROW + 16 * ks + 8 * lh]);
+        f[t] = *reinterpret_cast<const f16x8 *>(&bt[(cb + t * 32 + lr) * LDS_ROW + 16 * ks + 8 * lh]);
+    };
+    if constexpr (TN == 2) {
+      // One consumer wave per SIMD has nothing else to issue while it waits
+      // for LDS, about 200 cycles after the 256 of a k-step's MFMAs when the
+      // fragments are read k-step by k-step (an iteration took 2060 cycles
+      // for 1024 of MFMA work).  So A fragments are read two steps (4 MFMAs)
+      // and B fragments a k-step ahead of their use, in the 36 registers
+      // that 128 accumulators leave: 2048 x 28672 x 4096 559 -> 510 us, 512
+      // x 28672 x 4096 155 -> 143, 2048 x 6144 x 4096 148 -> 135, the same
+      // bits.  (Three steps ahead is no faster, and the smaller tiles lose
+      // 2-9 % this way: the reads of a whole k-step there are few.)
+      constexpr int NX = KS / 16 * TM;
+      f16x8 af[3], bf[2][TN];
+      read_b(bf[0], 0);
+      read_a(af[0], 0, 0);
+      read_a(af[1], 1 / TM, 1 % TM);
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int x = 0; x < NX; ++x) {
+        if (x % TM == 0 && x / TM + 1 < KS / 16) read_b(bf[(x / TM + 1) & 1], x / TM + 1);
+        if (x + 2 < NX) read_a(af[(x + 2) % 3], (x + 2) / TM, (x + 2) % TM);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < TN; ++t)
-          acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[t], acc[i][t], 0, 0, 0);
+          acc[x % TM][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[x % 3], bf[x / TM & 1][t],
+                                                                  acc[x % TM][t], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < KS / 16; ++ks) {
+        f16x8 af[TM], bf[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) read_a(af[i], ks, i);
+        read_b(bf, ks);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int t = 0; t < TN; ++t)
+            acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[t], acc[i][t], 0, 0, 0);
+      }
     }
     __syncthreads();
   }
