@@ -370,6 +370,17 @@ int q8_argmax(q8_ctx *ctx, q8_buf *a, uint64_t ox_f32, int64_t n, q8_buf *ids,
  * (the device side of n_cached += s, qwen3_mojo/src/qwen_q8.mojo:138). */
 int q8_pos_advance(q8_ctx *ctx, q8_buf *posbuf, uint64_t opos_i32, int64_t s);
 
+/* The start of a run of token steps in one launch on the stream, with no
+ * host synchronisation: the token id to ids[oid], the position (>= 0) to
+ * posbuf[opos] and, with w non-null, the embedding row of that id -- from the
+ * vocab packed rows of d at oemb of w, as q8_embed_gather -- to the d floats
+ * at ox of a.  id and pos are taken by value.  Stands for the host's writes of
+ * the id and n_cached and the embed of the first token
+ * (qwen3_mojo/src/qwen_q8.mojo:110-138). */
+int q8_token_begin(q8_ctx *ctx, q8_buf *ids, uint64_t oid_i32, int32_t id, q8_buf *posbuf,
+                   uint64_t opos_i32, int32_t pos, q8_buf *w, uint64_t oemb_u16, q8_buf *a,
+                   uint64_t ox_f32, int64_t d, int64_t vocab, int G, int scale_dtype);
+
 /* ---- HIP graphs ------------------------------------------------------------ */
 
 /* Capture every call issued on the context's stream between begin and end

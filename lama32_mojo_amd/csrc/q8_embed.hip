@@ -44,6 +44,38 @@ hipError_t launch_g(const GatherArgs &a, hipStream_t st) {
   return hipGetLastError();
 }
 
+// The start of a run of token steps: the token id and the position, given by
+// value, written to device memory and (emb non-null) that id's embedding row
+// gathered as embed_gather_kernel gathers it, in one launch.
+template <int G, int KIND>
+__global__ __launch_bounds__(256) void token_begin_kernel(int32_t id, int32_t *__restrict__ ids,
+                                                          int pos, int *__restrict__ posp,
+                                                          const uint8_t *__restrict__ emb,
+                                                          int64_t row_bytes, int64_t vocab,
+                                                          float *__restrict__ x, int64_t d) {
+  constexpr int SB = ScaleTraits<KIND>::bytes;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    ids[0] = id;
+    posp[0] = pos;
+  }
+  const int64_t c = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+  if (!emb || c >= d) return;
+  const bool ok = id >= 0 && id < vocab;
+  const uint8_t *row = emb + (ok ? id : 0) * row_bytes;
+  const float sc = ok ? load_scale<KIND>(row, c / G) : __builtin_nanf("");
+  const int8_t *codes = reinterpret_cast<const int8_t *>(row + (d / G) * SB);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) x[c + u] = ok ? (float)codes[c + u] * sc : sc;
+}
+
+template <int G, int KIND>
+hipError_t launch_begin_g(const TokenBeginArgs &a, hipStream_t st) {
+  const int64_t blocks = a.emb ? (a.d / 4 + 255) / 256 : 1;
+  hipLaunchKernelGGL((token_begin_kernel<G, KIND>), dim3((unsigned)blocks), dim3(256), 0, st, a.id,
+                     a.ids, a.pos, a.posp, a.emb, a.row_bytes, a.vocab, a.x, a.d);
+  return hipGetLastError();
+}
+
 // The token step's last launch: the argmax over the GEMV's per-workgroup
 // partials (value desc, row asc; k_argmax's result: index 0 when logits[0]
 // is NaN or no value exceeds it), written to ids[0]; the device position
@@ -130,6 +162,14 @@ hipError_t launch_finish_g(const ArgmaxFinishArgs &a, hipStream_t st) {
 }
 
 }  // namespace
+
+hipError_t launch_token_begin(const TokenBeginArgs &a, hipStream_t st) {
+  // (a table without rows is never read: every id is outside it)
+  if (a.G == 64 && a.kind == SCALE_F32) return launch_begin_g<64, SCALE_F32>(a, st);
+  if (a.G == 32 && a.kind == SCALE_F16) return launch_begin_g<32, SCALE_F16>(a, st);
+  if (a.G == 32 && a.kind == SCALE_F32) return launch_begin_g<32, SCALE_F32>(a, st);
+  return launch_begin_g<64, SCALE_F16>(a, st);
+}
 
 hipError_t launch_argmax_finish(const ArgmaxFinishArgs &a, hipStream_t st) {
   if (a.nblocks < 1 || a.nblocks > kArgmaxMaxBlocks) return hipErrorInvalidValue;

@@ -234,5 +234,18 @@ struct ArgmaxFinishArgs {
 };
 hipError_t launch_argmax_finish(const ArgmaxFinishArgs &a, hipStream_t st);
 hipError_t launch_pos_advance(int *pos, int s, hipStream_t st);
+// ids[0] = id and *posp = pos; with emb non-null, id's embedding row (d
+// floats; NaN for an id outside [0, vocab)) to x.
+struct TokenBeginArgs {
+  int32_t id;
+  int32_t *ids;
+  int pos;
+  int *posp;
+  const uint8_t *emb;    // packed table (vocab rows) or null
+  int64_t row_bytes, vocab, d;
+  int G, kind;
+  float *x;
+};
+hipError_t launch_token_begin(const TokenBeginArgs &a, hipStream_t st);
 
 }  // namespace q8

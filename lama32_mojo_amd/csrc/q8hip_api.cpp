@@ -1458,6 +1458,46 @@ int q8_pos_advance(q8_ctx *ctx, q8_buf *posbuf, uint64_t opos_i32, int64_t s) {
   return ok(ctx);
 }
 
+int q8_token_begin(q8_ctx *ctx, q8_buf *ids, uint64_t oid_i32, int32_t id, q8_buf *posbuf,
+                   uint64_t opos_i32, int32_t pos, q8_buf *w, uint64_t oemb_u16, q8_buf *a,
+                   uint64_t ox_f32, int64_t d, int64_t vocab, int G, int scale_dtype) {
+  if (int rc = check_ctx(ctx)) return rc;
+  if (!ids || !posbuf) return fail(ctx, Q8_ERR_ARG, "q8_token_begin: null buffer");
+  if (pos < 0) return fail(ctx, Q8_ERR_ARG, "q8_token_begin: position %d", (int)pos);
+  if (!fits(oid_i32, 1, 4, ids->size) || !fits(opos_i32, 1, 4, posbuf->size))
+    return fail(ctx, Q8_ERR_RANGE, "q8_token_begin: id or position offset exceeds its buffer");
+  uint64_t rs = 0;
+  if (w) {
+    if (!a) return fail(ctx, Q8_ERR_ARG, "q8_token_begin: null activation buffer");
+    if (int rc = check_layout(ctx, d, G, scale_dtype, "q8_token_begin")) return rc;
+    if (vocab < 0)
+      return fail(ctx, Q8_ERR_SHAPE, "q8_token_begin: vocab=%lld", (long long)vocab);
+    rs = (uint64_t)rowstride_u16(d, G, scale_dtype);
+    if (!fits(oemb_u16, (uint64_t)vocab * rs, 2, w->size))
+      return fail(ctx, Q8_ERR_RANGE, "q8_token_begin: table of %lld rows exceeds the weight buffer",
+                  (long long)vocab);
+    if (!fits(ox_f32, (uint64_t)d, 4, a->size))
+      return fail(ctx, Q8_ERR_RANGE, "q8_token_begin: row exceeds the activation buffer");
+  }
+  if (ctx->host_only) return fail(ctx, Q8_ERR_NODEVICE, "q8_token_begin: host-only context");
+  if (int rc = set_device(ctx)) return rc;
+  q8::TokenBeginArgs t;
+  t.id = id;
+  t.ids = reinterpret_cast<int32_t *>(bytes(ids, oid_i32 * 4));
+  t.pos = pos;
+  t.posp = reinterpret_cast<int *>(bytes(posbuf, opos_i32 * 4));
+  t.emb = w ? bytes(w, oemb_u16 * 2) : nullptr;
+  t.row_bytes = (int64_t)rs * 2;
+  t.vocab = vocab;
+  t.d = d;
+  t.G = G;
+  t.kind = scale_dtype;
+  t.x = w ? fptr(a, ox_f32) : nullptr;
+  hipError_t e = q8::launch_token_begin(t, ctx->stream);
+  if (e != hipSuccess) return hip_fail(ctx, e, "q8_token_begin launch");
+  return ok(ctx);
+}
+
 // ---- HIP graphs -------------------------------------------------------------------
 
 struct q8_graph {

@@ -584,12 +584,10 @@ class Q8Llama:
         position (the cached length) and, for the fused step, the first
         token's embedding row in the step's input."""
         self.capture_decode()
-        self.ids.upload(np.array([first_id], dtype=np.int32))
-        self.posbuf.upload(np.array([self.n_cached], dtype=np.int32))
-        if self.fuse:
-            q8hip.embed_gather(self.ctx, self.w.buf, self.w.o("model.embed_tokens.weight"),
-                               self.ids, 0, self.a.buf, self.graph_x, 1, self.cfg.hidden,
-                               self.cfg.vocab, self.G, self.scale)
+        emb = dict(w=self.w.buf, oemb_u16=self.w.o("model.embed_tokens.weight"), a=self.a.buf,
+                   ox_f32=self.graph_x, d=self.cfg.hidden, vocab=self.cfg.vocab, G=self.G,
+                   scale=self.scale) if self.fuse else {}
+        q8hip.token_begin(self.ctx, self.ids, 0, first_id, self.posbuf, 0, self.n_cached, **emb)
 
     def decode_steps(self, first_id: int, n: int) -> list[int]:
         """Greedy-decode n tokens starting from first_id at the current

@@ -115,6 +115,8 @@ SIGNATURES = {
     "q8_add": (_I, [_P, _P, _U64, _U64, _I64]),
     "q8_argmax": (_I, [_P, _P, _U64, _I64, _P, _U64]),
     "q8_pos_advance": (_I, [_P, _P, _U64, _I64]),
+    "q8_token_begin": (_I, [_P, _P, _U64, ctypes.c_int32, _P, _U64, ctypes.c_int32, _P, _U64, _P,
+                            _U64, _I64, _I64, _I, _I]),
     "q8_graph_begin": (_I, [_P]),
     "q8_graph_end": (_I, [_P, ctypes.POINTER(_P)]),
     "q8_graph_launch": (_I, [_P, _P]),
@@ -469,3 +471,16 @@ def argmax(ctx: Context, a: Buffer, ox: int, n: int, ids: Buffer, oid_i32: int) 
 
 def pos_advance(ctx: Context, posbuf: Buffer, opos_i32: int, s: int) -> None:
     ctx.check(ctx._lib.q8_pos_advance(ctx.h, posbuf.h, int(opos_i32), int(s)))
+
+
+def token_begin(ctx: Context, ids: Buffer, oid_i32: int, token: int, posbuf: Buffer,
+                opos_i32: int, pos: int, w: Buffer | None = None, oemb_u16: int = 0,
+                a: Buffer | None = None, ox_f32: int = 0, d: int = 0, vocab: int = 0,
+                G: int = 64, scale="f16") -> None:
+    """The token id and position to device memory and (with w) the token's
+    embedding row to ox_f32, in one launch: q8_token_begin."""
+    # (raises where the value does not fit an int32, as an int32 array does)
+    token, pos = (int(v) for v in np.array([token, pos], dtype=np.int32))
+    ctx.check(ctx._lib.q8_token_begin(ctx.h, ids.h, int(oid_i32), token, posbuf.h, int(opos_i32),
+                                      pos, _h(w), int(oemb_u16), _h(a), int(ox_f32), int(d),
+                                      int(vocab), int(G), scale_code(scale)))

@@ -316,6 +316,23 @@ def test_embed_validation(hctx):
     assert code_of(E, hctx, w, 0, ids, 0, a, 0, 4, 100, vocab)[0] == Q8_ERR_SHAPE
 
 
+def test_token_begin_validation(hctx):
+    d, vocab = 2048, 10
+    rs = q8hip.rowstride_u16(d)
+    w, a = hctx.alloc(2 * vocab * rs), hctx.alloc(4 * d)
+    ids, pos = hctx.alloc(4), hctx.alloc(8)
+    T = q8hip.token_begin
+    assert code_of(T, hctx, ids, 0, 3, pos, 1, 7, w, 0, a, 0, d, vocab)[0] == Q8_ERR_NODEVICE
+    assert code_of(T, hctx, ids, 0, 3, pos, 1, 7)[0] == Q8_ERR_NODEVICE
+    assert code_of(T, hctx, ids, 1, 3, pos, 1, 7)[0] == Q8_ERR_RANGE
+    assert code_of(T, hctx, ids, 0, 3, pos, 2, 7)[0] == Q8_ERR_RANGE
+    assert code_of(T, hctx, ids, 0, 3, pos, 0, -1)[0] == Q8_ERR_ARG
+    assert code_of(T, hctx, ids, 0, 3, pos, 0, 7, w, 0, a, 1, d, vocab)[0] == Q8_ERR_RANGE
+    assert code_of(T, hctx, ids, 0, 3, pos, 0, 7, w, 0, a, 0, d, vocab + 1)[0] == Q8_ERR_RANGE
+    assert code_of(T, hctx, ids, 0, 3, pos, 0, 7, w, 0, a, 0, 100, vocab)[0] == Q8_ERR_SHAPE
+    assert code_of(T, hctx, ids, 0, 3, pos, 0, 7, w, 0, None, 0, d, vocab)[0] == Q8_ERR_ARG
+
+
 def test_null_handles():
     lib = q8hip.lib()
     assert lib.q8_linear(None, None, 0, None, 0, 0, 1, 64, 1, 64, 1) == Q8_ERR_ARG

@@ -22,7 +22,7 @@ import pytest
 from lama32_mojo_amd import model as gm
 from lama32_mojo_amd import q8hip
 from oracle import model_oracle as mo
-from oracle.q8_oracle import f32_to_bf16_bits, max_rel_err
+from oracle.q8_oracle import f32_to_bf16_bits, max_rel_err, pack_q8_np
 
 sys.path.insert(0, __file__.rsplit("/", 1)[0])
 from test_model_oracle import qwen_tiny, tiny_model  # noqa: E402
@@ -983,3 +983,31 @@ def test_fused_graph_decode_equals_unfused_graph(ctx):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("G,scale", [(64, "f16"), (32, "f32")])
+@pytest.mark.parametrize("d", [64, 1024, 4096])
+@pytest.mark.parametrize("token", [0, 36, -1, 37])
+def test_token_begin_equals_uploads_and_gather(ctx, G, scale, d, token):
+    """q8_token_begin leaves what writing the id and the position and then
+    q8_embed_gather leave: the same bits, NaN rows for ids outside the table,
+    the words beside the id and the position untouched."""
+    say("token begin", G, scale, d, token)
+    vocab = 37
+    pk = pack_q8_np(np.random.default_rng(d).standard_normal((vocab, d)).astype(np.float32), G,
+                    scale)
+    w = ctx.alloc(pk.nbytes)
+    w.upload(pk)
+    a = arena(ctx, 2 * d)
+    ids, pb = ctx.alloc(16), ctx.alloc(16)
+    for b in (ids, pb):
+        b.upload(np.full(4, 77, np.int32))
+    q8hip.token_begin(ctx, ids, 1, token, pb, 2, 1234, w, 0, a, 0, d, vocab, G, scale)
+    q8hip.embed_gather(ctx, w, 0, ids, 1, a, d, 1, d, vocab, G, scale)
+    x = get(a, 0, (2, d))
+    assert np.array_equal(x[0], x[1], equal_nan=True)
+    assert np.all(np.isnan(x)) == (token in (-1, 37))
+    assert list(ids.download((4,), np.int32)) == [77, token, 77, 77]
+    assert list(pb.download((4,), np.int32)) == [77, 77, 1234, 77]
+    for b in (w, a, ids, pb):
+        b.free()
