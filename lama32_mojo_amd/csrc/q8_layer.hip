@@ -991,11 +991,21 @@ __global__ __launch_bounds__(HD) void attn_merge_kernel(const float *__restrict_
   const float f = lane < active ? expf(mx - big) : 0.0f;
   const float l = wave_sum(lane < active ? l_lane * f : 0.0f);
   float o = 0.0f;
+  // All NX splits active: unrolled, against the indexed loop 32 heads of 128
+  // at 4000 keys 10.4 -> 9.7 us, at 16000 20.1 -> 19.3; unrolled with a select
+  // per record, which serves every count, 9.9 and 19.5, and at few splits no
+  // faster than the loop.
+  if (active == NX) {
 #pragma unroll
-  for (int x = 0; x < NX; ++x) {
-    // (a record past the active ones was not written: a select)
-    const float fx = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), x));
-    o = __builtin_fmaf(x < active ? ov[x] : 0.0f, fx, o);
+    for (int x = 0; x < NX; ++x) {
+      const float fx = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), x));
+      o = __builtin_fmaf(ov[x], fx, o);
+    }
+  } else {   // ov[x]: indexed register reads (a record past the active ones was not written)
+    for (int x = 0; x < active; ++x) {
+      const float fx = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), x));
+      o = __builtin_fmaf(ov[x], fx, o);
+    }
   }
   out[h * HD + d] = o / l;
 }
