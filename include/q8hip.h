@@ -119,10 +119,13 @@ int q8_quantize_pack(q8_ctx *ctx, q8_buf *src, uint64_t src_off, int src_dtype,
  * and 2 .. 4 rows f32 4x4-block MFMA, both with f32 products of x and the
  * codes; 5 .. 31 rows split each x into two bf16 terms hi + lo (x - hi - lo
  * below 2^-17 |x|, so x is carried to that bound, not exactly) whose
- * products with the codes are exact on bf16 MFMA; all three stay within
+ * products with the codes are exact on bf16 MFMA; 17 .. 31 rows of m >= 4096
+ * codes, and two rows and up whose packed rows or x are not 16-byte aligned,
+ * carry x as two binary16 terms after a power-of-two row scaling (to
+ * 2^-22 |x|), again with exact products; all of these stay within
  * 1e-5 of float64.  s >= 32 runs the dequant-GEMM on f16 MFMA (binary16 x
  * rows after a power-of-two scaling, binary16 q * s), whose max-rel-err
- * stays near 2e-4. */
+ * stays near 2e-4 (aligned operands only). */
 int q8_linear(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *a,
               uint64_t ox_f32, uint64_t oy_f32, int64_t s, int64_t m, int64_t n,
               int G, int scale_dtype);
@@ -132,6 +135,8 @@ int q8_linear(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *a,
  * dequant-GEMM on f16 MFMA: each x row scaled by a power of two into
  * binary16 (exact for bf16 values), weights q * s rounded once to binary16
  * (twice with f32 scales), f32 accumulation; max-rel-err stays near 2e-4.
+ * Operands that are not 16-byte aligned keep the codes exact and scale each
+ * group's f32 partial instead (within 1e-5 of float64).
  * No reference counterpart (the reference is W8A32 only); it is the
  * M = 512 bf16-activation prefill case. */
 int q8_linear_bf16act(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *x,

@@ -336,13 +336,15 @@ __device__ __forceinline__ f16x8 dequant8(uint32_t d0, uint32_t d1, f16x2 s2) {
 // Measured on the 1B / 8B prefill shapes against one 8-wave role-free form
 // (every wave staging, dequantizing its own columns in registers and
 // issuing MFMAs, two K parities): 512x16384x2048 63.2 -> 55.4 us,
-// 2048x14336x4096 342 -> 307 us, 2048x4096x14336 309 -> 276 us.  Alone,
-// the consumers reach 1.45 PFLOP/s on 2048x14336x4096 and the producers
-// take 225 us: the producers set the pace (their loads, dequantizing VALU
-// and LDS writes run in lockstep phases between the barriers; LDS takes
-// about 385 GB/s of 16-byte reads and 174 GB/s of 16-byte writes per CU
-// here), and 4 producer waves instead of 8, or 3-4 register stages instead
-// of 2, were slower or equal.
+// 2048x14336x4096 342 -> 307 us, 2048x4096x14336 309 -> 276 us; since then
+// the producers keep two iterations of loads in flight, the 256-wide tiles
+// read fragments ahead of their MFMAs and the epilogue has no branches:
+// 512x16384x2048 42.5 us, 2048x28672x4096 507 us (0.95 PFLOP/s).  Bound: the
+// stage hand-over per iteration (the producers' dequantizing and LDS writes
+// run in lockstep phases between the barriers; LDS takes about 385 GB/s of
+// 16-byte reads and 174 GB/s of 16-byte writes per CU here).  4 producer
+// waves instead of 8, or 3-4 register stages instead of 2, were slower or
+// equal.
 constexpr int kIterCodes = 64;     // k per iteration (128 on 64-row tiles)
 constexpr int kProducerWaves = 8;
 constexpr int kStages = 2;         // register stages of the producers

@@ -47,7 +47,8 @@ struct LinearArgs {
   const float *res = nullptr;
   float *hout = nullptr;
 };
-// Decode path (s small, f32 x): VALU GEMV.
+// Decode path (s = 1, f32 x, any alignment): VALU GEMV; more rows only as the
+// last resort of unaligned operands that fit no scratch.
 hipError_t launch_gemv(const LinearArgs &a, hipStream_t st);
 // One-row GEMV with its neighbours folded in (decode step, s = 1).
 // Prologue (how x is read):
@@ -89,7 +90,8 @@ hipError_t launch_gemm(const LinearArgs &a, uint16_t *x16, int *ex, int *ew, boo
 // y[i] = sum over z < splits of ws[z * count + i] (split-K partial sums).
 hipError_t launch_splitk_reduce(const float *ws, float *y, int64_t count, int splits,
                                 hipStream_t st);
-// Small batches (s <= 32, f32 x; the C ABI sends it 5 <= s < 32): bf16 MFMA
+// Small batches (s <= 32, f32 x; the C ABI sends it 5 <= s < 32, from 17 rows
+// on only where a row has fewer than 4096 codes or fits no scratch): bf16 MFMA
 // over zero-padded 16-row tiles with x split into two bf16 terms.
 hipError_t launch_skinny(const LinearArgs &a, hipStream_t st);
 // A few rows (2 <= s <= kSkinny4MaxRows, f32 x): f32 4x4 MFMA blocks over
@@ -130,7 +132,7 @@ hipError_t launch_rope_kv(float *q, float *k, const float *v, __half *kc, __half
 struct AttnArgs {
   const float *q;        // [s, nheads * head_dim], rotated, row i at q + i * ldq
   const __half *kc, *vc; // [maxlen, nkv * head_dim]
-  float *part;           // scratch (s < kPrefillMinRows only):
+  float *part;           // scratch (s < kPrefillMinRows without mfma_ok):
                          //   s * nheads * nsplit * (head_dim + 2) floats
   float *out;            // [s, nheads * head_dim]
   int s, nheads, nkv, head_dim, nsplit;
@@ -143,9 +145,10 @@ struct AttnArgs {
   int64_t ws_floats = 0;
   bool mfma_ok = false;  // fewer rows may take the MFMA pass (16-byte aligned q, out, rows)
 };
-// Row counts from which attention runs as one MFMA pass per (row block, KV
-// head) with no scratch; below it, as (KV head, 64-key split) partials
-// merged by a second kernel.
+// Row counts from which attention always runs as MFMA passes per (row block,
+// KV head), over key splits merged by a second kernel where the row blocks
+// leave the chip idle; fewer rows do too with mfma_ok, else as (KV head,
+// 64-key split) partials merged by a second kernel.
 constexpr int kPrefillMinRows = 16;
 // Causal GQA attention of s query rows at positions pos0 .. pos0+s-1 over
 // cache rows 0 .. pos0+i; nsplit = ceil(maxlen / 64).

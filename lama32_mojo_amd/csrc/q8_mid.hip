@@ -21,7 +21,9 @@
 // + m bytes, so most widths that are no multiple of 512 at G = 64 with f16
 // scales), against one wave per output with one code per lane and load:
 // 200 x 1600 x 4800 1030 -> 28 us, 512 x 11008 x 4096 24390 -> 133 us, 16 x
-// 11008 x 4096 777 -> 24 us, 2 x 1600 x 4800 17 -> 12.5 us.
+// 11008 x 4096 777 -> 24 us, 2 x 1600 x 4800 17 -> 12.5 us; and 17 .. 31
+// aligned rows of 4096 codes or more (31 x 4096 x 24576 65 -> 44 us; the line
+// is drawn in the dispatch).
 //
 // Layout: a workgroup owns 32 RT rows x 32 C KW columns, wave w 32 C
 // columns of them, and a range of 64-code units of K.  Per phase of PU units
