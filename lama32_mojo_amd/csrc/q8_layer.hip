@@ -281,6 +281,49 @@ __host__ __device__ inline int split_tiles(int ntiles, int nz) {
   const int t = (ntiles + nz - 1) / nz;
   return ntiles - t >= 6 ? t : ntiles;
 }
+// One (row, head) over keys j0 .. j1-1 by one wave in f32, reading no other
+// key: o of dims lane (and lane + 64) unnormalised, with the maximum m of the
+// scores in the log2 domain and the sum l of exp2(score - m).
+template <int HD>
+__device__ __forceinline__ void attn_row_f32(const float *__restrict__ q,
+                                             const __half *__restrict__ kc,
+                                             const __half *__restrict__ vc, int kvdim, int j0,
+                                             int j1, int lane, float (&o)[HD / 64], float &m,
+                                             float &l) {
+  const float cs = 1.44269504088896341f / sqrtf((float)HD);
+  m = -INFINITY;
+  l = 0.0f;
+#pragma unroll
+  for (int e = 0; e < HD / 64; ++e) o[e] = 0.0f;
+  for (; j0 < j1; j0 += 64) {
+    const int nk = min(64, j1 - j0);
+    float sc = -INFINITY;
+    if (lane < nk) {
+      const __half *kr = kc + (int64_t)(j0 + lane) * kvdim;
+      sc = 0.0f;
+#pragma unroll 4
+      for (int d = 0; d < HD; ++d) sc = __builtin_fmaf(q[d], __half2float(kr[d]), sc);
+      sc *= cs;
+    }
+    const float mn = fmaxf(m, wave_max(sc));
+    const float ms = mn == -INFINITY ? 0.0f : mn;  // (nothing but scores of -inf so far)
+    const float alpha = exp2f(m - ms);
+    const float p = lane < nk ? exp2f(sc - ms) : 0.0f;
+    l = __builtin_fmaf(l, alpha, wave_sum(p));
+    m = mn;
+#pragma unroll
+    for (int e = 0; e < HD / 64; ++e) o[e] *= alpha;
+    for (int t = 0; t < nk; ++t) {
+      const float pt =
+          __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), t));
+      const __half *vr = vc + (int64_t)(j0 + t) * kvdim + lane;
+#pragma unroll
+      for (int e = 0; e < HD / 64; ++e)
+        o[e] = __builtin_fmaf(pt, __half2float(vr[64 * e]), o[e]);
+    }
+  }
+}
+
 template <int HD, int GRP, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_prefill_kernel(const float *__restrict__ q,
@@ -509,7 +552,23 @@ void attn_prefill_kernel(const float *__restrict__ q,
       }
   }
   l += __shfl_xor(l, 32);
-  if (i < s) {
+  // The MFMAs multiply every key of a tile into every column: 0 times an
+  // infinite or NaN v of a key that the column's row must not see is NaN, and
+  // so is an infinity of a key that it sees times the hi and lo halves of p
+  // or q.  A sum that once was not finite stays so (alpha 0 times infinity
+  // is NaN), so one look at the sums here finds these columns, and only
+  // they are formed again from their own keys alone, in f32.  (A cache of
+  // finite f32 rows holds infinities where |v| > 65504.)  The look costs 0.1
+  // us a call (16 rows, no cache: 7.3 -> 7.4; 2048 rows: 85.9 both).
+  float chk = 0.0f * l;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) chk = __builtin_fmaf(o[t][v], 0.0f, chk);
+  chk += __shfl_xor(chk, 32);
+  const bool bad = chk != 0.0f;
+  float2 *ml = reinterpret_cast<float2 *>(part + (int64_t)gridDim.z * s * qdim);
+  if (i < s && !bad) {
     const float il = apart ? 1.0f / 16384.0f : 1.0f / (l * 16384.0f);
     const int64_t rec = (int64_t)blockIdx.z * s + i;
     float *orow = (apart ? part + rec * qdim : out + (int64_t)i * qdim) + head * HD + 4 * hf;
@@ -522,10 +581,19 @@ void attn_prefill_kernel(const float *__restrict__ q,
         for (int c = 0; c < 4; ++c) r[c] = o[d][4 * vb + c] * il;
         *reinterpret_cast<f32x4 *>(orow + 32 * d + 8 * vb) = r;
       }
-    if (apart && hf == 0) {
-      float2 *ml = reinterpret_cast<float2 *>(part + (int64_t)gridDim.z * s * qdim);
-      ml[rec * nheads + head] = make_float2(m, l);
-    }
+    if (apart && hf == 0) ml[rec * nheads + head] = make_float2(m, l);
+  }
+  for (uint32_t left = (uint32_t)__builtin_amdgcn_ballot_w64(i < s && bad); left; left &= left - 1) {
+    const int c = __builtin_ctz(left);           // column c: lanes c and c + 32
+    const int ci = row0 + w * PW + c / GRP, ch = g * GRP + c % GRP;
+    float oc[HD / 64], mc, lc;
+    attn_row_f32<HD>(q + (int64_t)ci * ldq + ch * HD, kc + g * HD, vc + g * HD, kvdim, kt0 * BK,
+                     min(kt1 * BK, min(pos0 + ci + 1, maxlen)), lane, oc, mc, lc);
+    const int64_t rec = (int64_t)blockIdx.z * s + ci;
+    float *orow = (apart ? part + rec * qdim : out + (int64_t)ci * qdim) + ch * HD + lane;
+#pragma unroll
+    for (int e = 0; e < HD / 64; ++e) orow[64 * e] = apart ? oc[e] : oc[e] / lc;
+    if (apart && lane == 0) ml[rec * nheads + ch] = make_float2(mc, lc);
   }
 }
 
@@ -564,10 +632,11 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float *__
       a[u] = ml[z * rows + r];
       v[u] = *reinterpret_cast<const f32x4 *>(part + (z * rows + r) * HD + d);
     }
-    // (split 0 holds key 0, which every row sees: the maximum is finite)
+    // (nothing but scores of -inf so far: any finite reference will do)
     float mx = m;
 #pragma unroll
     for (int u = 0; u < 8; ++u) mx = fmaxf(mx, z0 + u < nz ? a[u].x : -INFINITY);
+    mx = mx == -INFINITY ? 0.0f : mx;
     const float f0 = exp2f(m - mx);
     l *= f0;
     o *= f0;

@@ -203,6 +203,54 @@ def test_attention_key_splits(ctx, head_dim, nh, nkv, s, pos0, maxlen, shift):
         b.free()
 
 
+@pytest.mark.parametrize("head_dim,nh,nkv", [(128, 8, 2), (64, 4, 2), (64, 2, 2)])
+@pytest.mark.parametrize("s", [1, 2, 15, 16, 40])
+@pytest.mark.parametrize("pos0", [20, 1500])
+def test_attention_non_finite_cache_rows(ctx, head_dim, nh, nkv, s, pos0):
+    """Infinities and NaN in K and V of rows that some or all query rows see,
+    served whole and split: each row is its own keys' softmax and no other's
+    (a row before an infinite v keeps its finite values), an infinite v gives
+    infinities and no NaN, a score of -inf counts nothing."""
+    say("attention non-finite", head_dim, nh, nkv, s, pos0)
+    rng = np.random.default_rng(s + pos0 + head_dim)
+    n, maxlen = pos0 + s, pos0 + s + 3
+    qd, kvd = nh * head_dim, nkv * head_dim
+    mid, last = pos0 + s // 2, n - 1
+    for rows in ([("v", mid, 3, np.inf), ("v", last, head_dim + 5, np.nan)],
+                 [("v", 7, 2, -np.inf), ("v", mid, 9, np.inf)],
+                 [("k", mid, 1, np.nan)], [("k", 9, 1, np.inf), ("k", mid, head_dim, -np.inf)],
+                 [("k", j, head_dim - 1, np.inf) for j in range(8)]):
+        cache = np.full((2, maxlen, kvd), np.nan, np.float16)
+        cache[0, :n] = rng.standard_normal((n, kvd)) * 0.7
+        cache[1, :n] = rng.standard_normal((n, kvd))
+        for what, j, d, value in rows:
+            cache["kv".index(what), j, d] = value
+        q = rng.standard_normal((s, qd)).astype(np.float32)
+        kv = ctx.alloc(cache.nbytes)
+        kv.upload(cache)
+        oy = s * qd
+        osc = oy + s * qd
+        a = arena(ctx, osc + q8hip.attention_scratch_floats(s, nh, head_dim, maxlen) + 4)
+        put(a, 0, q)
+        q8hip.attention(ctx, a, 0, kv, 0, maxlen * kvd, maxlen, oy, osc, s, pos0, nh, nkv, head_dim)
+        got = get(a, oy, (s, nh, head_dim))
+        c = cache.astype(np.float64).reshape(2, maxlen, nkv, head_dim)
+        with np.errstate(all="ignore"):
+            for i in range(s):
+                for h in range(nh):
+                    k, v = c[:, :pos0 + i + 1, h * nkv // nh]
+                    sc = k @ q[i, h * head_dim:(h + 1) * head_dim].astype(np.float64)
+                    p = np.exp((sc - np.fmax.reduce(sc)) / np.sqrt(head_dim))
+                    ref = (p[:, None] * v).sum(0) / p.sum()
+                    ok = np.isfinite(ref)
+                    assert np.array_equal(got[i, h][~ok], ref[~ok].astype(np.float32),
+                                          equal_nan=True), (rows, i, h)
+                    assert np.allclose(got[i, h][ok], ref[ok], rtol=0,
+                                       atol=1e-5 * np.abs(ref[ok]).max(initial=0.0)), (rows, i, h)
+        for b in (a, kv):
+            b.free()
+
+
 @pytest.mark.parametrize("head_dim,nh,nkv,s", [(64, 8, 2, 3), (128, 32, 8, 48),
                                                (64, 32, 8, 130)])
 def test_stacked_qkv_rows_equal_dense(ctx, head_dim, nh, nkv, s):
