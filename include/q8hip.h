@@ -71,7 +71,14 @@ int q8_create(int device_ordinal, q8_ctx **out);
 void q8_destroy(q8_ctx *ctx);
 
 /* Run subsequent calls on an existing hipStream_t (NULL: the context's own
- * stream).  The caller keeps ownership of the stream. */
+ * stream).  The caller keeps ownership of the stream.  Calls on different
+ * streams are not ordered, except that one that uses the context's scratch
+ * (q8_linear of more than 4 rows or of unaligned ones, q8_linear_bf16act, _swiglu
+ * and _rmsnorm, q8_head_argmax, q8_decode_attention, q8_attention from 16
+ * rows on, q8_graph_launch) starts behind the last such call on another
+ * stream; for that, a stream stays valid until another one is set, or
+ * until q8_sync has returned on it.  A graph that the caller captured and
+ * launches by itself is not seen by this. */
 int q8_set_stream(q8_ctx *ctx, void *hip_stream);
 void *q8_get_stream(q8_ctx *ctx);
 
@@ -318,11 +325,11 @@ uint64_t q8_attention_scratch_floats(int64_t s, int nheads, int head_dim,
  * 1/sqrt(head_dim)) -- k_scores, k_softmax_rows and k_att_out
  * (src/llama_common.mojo:402-473) with their score buffer replaced by an
  * online softmax: one MFMA pass per (16..128-row block, KV head), whose keys
- * are split over several blocks where few rows meet a long cache (the split
- * records live in the context's workspace, so calls on one context must not
- * overlap).  Below 16 rows operands that are not 16-byte aligned take
- * per-split partials in q8_attention_scratch_floats() floats at oscratch
- * (oscratch is unused when that is 0).  head_dim 64 or
+ * are split over several blocks where few rows meet a long cache; the split
+ * records live in the context's scratch, below 16 rows in the
+ * q8_attention_scratch_floats() floats at oscratch (unused when that is 0).
+ * Below 16 rows operands or scratch that are not 16-byte aligned take one
+ * block per (KV head, 64 keys, row) instead.  head_dim 64 or
  * 128, nheads / nkv in {1, 2, 4, 8}.  Position as in q8_rope_kv.  Row i of q
  * at oq + i*ldq (ldq = 0: nheads*head_dim, dense); out is dense.  From
  * s = 16 on, q and out must start 16-byte aligned and ldq be a multiple of 4
@@ -341,8 +348,7 @@ int q8_attention(q8_ctx *ctx, q8_buf *a, uint64_t oq_f32, q8_buf *kv,
  * attention of the token over rows 0 .. pos0 into out at oy (as
  * q8_attention), in two launches (context splits, then their merge).  q and
  * k in the arena are left as they were.  The split records live in the
- * context's workspace, so calls on one context must not overlap (they do
- * not when issued on its stream).  head_dim 64 or 128, nheads / nkv in
+ * context's scratch (q8_set_stream).  head_dim 64 or 128, nheads / nkv in
  * {1, 2, 4, 8}; a cache block must stay under 2 GiB; position as in
  * q8_rope_kv.
  * Replaces the per-token attention of run_layer_q8 (src/llama_q8.mojo:171-205:

@@ -140,7 +140,7 @@ struct AttnArgs {
   int pos0;
   int maxlen;            // cache rows; positions past it are clamped
   int64_t ldq;           // q row stride in floats (nheads * head_dim when dense)
-  // scratch of the MFMA pass's key splits (null: no split)
+  // scratch of the MFMA pass's key splits, 16-byte aligned (null: no split)
   float *ws = nullptr;
   int64_t ws_floats = 0;
   bool mfma_ok = false;  // fewer rows may take the MFMA pass (16-byte aligned q, out, rows)

@@ -26,15 +26,25 @@ struct q8_ctx {
   hipStream_t own = nullptr;
   hipStream_t stream = nullptr;
   std::string err;
-  // Split-K workspace of the prefill GEMM (partial sums).  A split only
+  // Split-K workspace of the linears (partial sums).  A GEMM split only
   // happens while tiles x splits stay within 256 workgroups of 64 x 128
   // outputs, so 2 Mi floats always suffice; 4 Mi leaves room.
-  // The decode attention's partial records use it too: both run in stream
-  // order on this context.
+  // The split records of the attention (decode, and prompts of 16 rows and
+  // up) and the vocabulary head's argmax partials use it too.
   float *gemm_ws = nullptr;
-  // Binary16 copy of the activation rows of a prefill GEMM and their
-  // power-of-two factors (launch_gemm); longer inputs run in row chunks.
+  // Activation rows of a prefill GEMM as binary16 with their power-of-two
+  // factors (launch_gemm), or as MFMA fragments (launch_mid); longer inputs
+  // run in row chunks.
   void *act16 = nullptr;
+  // Order of the uses of gemm_ws and act16 over the streams that q8_set_stream
+  // moves the context between (with_scratch).  The event is recorded when a
+  // stream is left, not at each use, so a program that stays on one stream,
+  // its own or the context's, records nothing (an event per call: 8 x 2048 x
+  // 2048 5.3 -> 9.0 us).
+  hipEvent_t used_ev = nullptr;
+  bool used = false;       // used on `stream` since it was set, the last mark or q8_sync
+  bool marked = false;     // used_ev marks a use
+  bool wait = false;       // `stream` has not waited for used_ev since it was set
   // Pinned staging for file -> device uploads (q8_st_upload): two halves,
   // allocated on first use.
   void *stage = nullptr;
@@ -108,6 +118,42 @@ int set_device(q8_ctx *ctx) {
   return Q8_OK;
 }
 
+// A stream on which no event can be recorded or waited for: one that is being
+// captured, or a caller's that no longer exists.
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// Marks the uses of the scratch on `stream` so far.  (A stream that is being
+// captured cannot be marked; its uses before the capture were when it began.)
+hipError_t mark_use(q8_ctx *ctx) {
+  if (!ctx->used) return hipSuccess;
+  if (!capturing(ctx->stream)) {
+    const hipError_t e = hipEventRecord(ctx->used_ev, ctx->stream);
+    if (e != hipSuccess) return e;
+    ctx->marked = true;
+  }
+  ctx->used = false;
+  return hipSuccess;
+}
+
+// Runs `launch`, which queues work that uses the scratch, behind the marked
+// use on another stream.  Calls recorded into a graph do not wait:
+// q8_graph_launch does so for the whole graph.
+template <class F>
+hipError_t with_scratch(q8_ctx *ctx, F launch) {
+  if (ctx->wait && !capturing(ctx->stream)) {
+    hipError_t e = hipStreamWaitEvent(ctx->stream, ctx->used_ev, 0);
+    if (e != hipSuccess) return e;
+    ctx->wait = false;
+  }
+  if (!ctx->wait) ctx->used = true;
+  return launch();
+}
+
 uint8_t *bytes(q8_buf *b, uint64_t off) {
   return static_cast<uint8_t *>(b->ptr) + off;
 }
@@ -153,7 +199,9 @@ int q8_create(int device_ordinal, q8_ctx **out) {
     }
     e = hipSetDevice(device_ordinal);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->own, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->used_ev, hipEventDisableTiming);
     if (e != hipSuccess) {
+      if (ctx->own) (void)hipStreamDestroy(ctx->own);
       delete ctx;
       return fail(nullptr, Q8_ERR_HIP, "q8_create: %s", hipGetErrorString(e));
     }
@@ -166,6 +214,7 @@ int q8_create(int device_ordinal, q8_ctx **out) {
       if (ctx->gemm_ws) (void)hipFree(ctx->gemm_ws);
       if (ctx->act16) (void)hipFree(ctx->act16);
       (void)hipStreamDestroy(ctx->own);
+      (void)hipEventDestroy(ctx->used_ev);
       delete ctx;
       return fail(nullptr, Q8_ERR_NOMEM, "q8_create: cannot allocate the GEMM workspace");
     }
@@ -185,6 +234,7 @@ void q8_destroy(q8_ctx *ctx) {
     }
     if (ctx->gemm_ws) (void)hipFree(ctx->gemm_ws);
     if (ctx->act16) (void)hipFree(ctx->act16);
+    if (ctx->used_ev) (void)hipEventDestroy(ctx->used_ev);
     if (ctx->stage) (void)hipHostFree(ctx->stage);
     for (hipEvent_t &ev : ctx->stage_ev)
       if (ev) (void)hipEventDestroy(ev);
@@ -195,7 +245,15 @@ void q8_destroy(q8_ctx *ctx) {
 int q8_set_stream(q8_ctx *ctx, void *hip_stream) {
   if (int rc = check_ctx(ctx)) return rc;
   if (ctx->host_only) return fail(ctx, Q8_ERR_NODEVICE, "q8_set_stream: host-only context");
-  ctx->stream = hip_stream ? static_cast<hipStream_t>(hip_stream) : ctx->own;
+  hipStream_t next = hip_stream ? static_cast<hipStream_t>(hip_stream) : ctx->own;
+  if (next == ctx->stream) return ok(ctx);
+  if (ctx->used) {
+    if (int rc = set_device(ctx)) return rc;
+    hipError_t e = mark_use(ctx);
+    if (e != hipSuccess) return hip_fail(ctx, e, "q8_set_stream");
+  }
+  ctx->stream = next;
+  ctx->wait = ctx->marked;
   return ok(ctx);
 }
 
@@ -207,6 +265,7 @@ int q8_sync(q8_ctx *ctx) {
   if (int rc = set_device(ctx)) return rc;
   hipError_t e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_sync");
+  ctx->used = false;
   return ok(ctx);
 }
 
@@ -482,7 +541,7 @@ hipError_t run_gemm_in(q8::LinearArgs la, void *act16, int64_t bytes, hipStream_
 
 hipError_t run_gemm(q8_ctx *ctx, q8::LinearArgs la) {
   attach_gemm_workspace(ctx, la);
-  return run_gemm_in(la, ctx->act16, kAct16Bytes, ctx->stream);
+  return with_scratch(ctx, [&] { return run_gemm_in(la, ctx->act16, kAct16Bytes, ctx->stream); });
 }
 
 // Device memory a W8A32 linear may use besides its inputs and outputs: the
@@ -517,8 +576,13 @@ hipError_t dispatch_linear(q8::LinearArgs la, const Scratch &sc, hipStream_t st)
   return q8::launch_skinny(la, st);
 }
 
-Scratch ctx_scratch(q8_ctx *ctx) {
-  return Scratch{ctx->gemm_ws, kGemmWsFloats, ctx->act16, kAct16Bytes};
+// The context's linear: one row, and aligned rows up to the 4x4-block
+// kernel's, use no scratch.
+hipError_t ctx_linear(q8_ctx *ctx, const q8::LinearArgs &la) {
+  const Scratch sc{ctx->gemm_ws, kGemmWsFloats, ctx->act16, kAct16Bytes};
+  auto launch = [&] { return dispatch_linear(la, sc, ctx->stream); };
+  if (la.s < kSkinnyMinRows || (la.s <= q8::kSkinny4MaxRows && gemm_aligned(la))) return launch();
+  return with_scratch(ctx, launch);
 }
 
 }  // namespace
@@ -555,7 +619,7 @@ int q8_linear(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *a, uint64_t ox_f
   la.n = n;
   la.G = G;
   la.kind = scale_dtype;
-  hipError_t e = dispatch_linear(la, ctx_scratch(ctx), ctx->stream);
+  hipError_t e = ctx_linear(ctx, la);
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_linear launch");
   return ok(ctx);
 }
@@ -599,7 +663,7 @@ int q8_linear_bf16act(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *x, uint6
   if (gemm_aligned(la))
     e = run_gemm(ctx, la);
   else
-    e = run_unaligned(la, ctx->act16, kAct16Bytes, ctx->stream);
+    e = with_scratch(ctx, [&] { return run_unaligned(la, ctx->act16, kAct16Bytes, ctx->stream); });
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_linear_bf16act launch");
   return ok(ctx);
 }
@@ -1047,18 +1111,15 @@ int q8_head_argmax(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, uint64_t onorm_u16,
   f.eps = eps;
   f.res = nullptr;
   f.part = ctx->gemm_ws;   // 2 x 8192 words of partials, read by the second launch
-  int grid = 0;
+  int grid = 0;   // set by the first launch
   f.grid_out = &grid;
   if (!q8::gemv_fused_supported(f))
     return fail(ctx, Q8_ERR_UNSUPPORTED, "q8_head_argmax: m=%lld (needs m <= 16384, m %% 32 == 0, "
                 "16-byte aligned rows and x, 8-byte aligned norm weights)", (long long)m);
   if (ctx->host_only) return fail(ctx, Q8_ERR_NODEVICE, "q8_head_argmax: host-only context");
   if (int rc = set_device(ctx)) return rc;
-  hipError_t e = q8::launch_gemv_fused(f, ctx->stream);
-  if (e != hipSuccess) return hip_fail(ctx, e, "q8_head_argmax launch");
   q8::ArgmaxFinishArgs fa;
   fa.part = ctx->gemm_ws;
-  fa.nblocks = grid;
   fa.logits = la.y;
   fa.ids = reinterpret_cast<int32_t *>(bytes(ids, oid_i32 * 4));
   fa.pos = posbuf ? reinterpret_cast<int *>(bytes(posbuf, opos_i32 * 4)) : nullptr;
@@ -1070,8 +1131,13 @@ int q8_head_argmax(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, uint64_t onorm_u16,
   fa.G = G;
   fa.kind = scale_dtype;
   fa.xnext = gather ? fptr(a, onext_f32) : nullptr;
-  e = q8::launch_argmax_finish(fa, ctx->stream);
-  if (e != hipSuccess) return hip_fail(ctx, e, "q8_head_argmax finish launch");
+  hipError_t e = with_scratch(ctx, [&] {
+    const hipError_t first = q8::launch_gemv_fused(f, ctx->stream);
+    if (first != hipSuccess) return first;
+    fa.nblocks = grid;
+    return q8::launch_argmax_finish(fa, ctx->stream);
+  });
+  if (e != hipSuccess) return hip_fail(ctx, e, "q8_head_argmax launch");
   return ok(ctx);
 }
 
@@ -1292,15 +1358,23 @@ int q8_attention(q8_ctx *ctx, q8_buf *a, uint64_t oq_f32, q8_buf *kv, uint64_t o
   aa.pos0 = (int)pos0;
   aa.maxlen = (int)maxlen;
   aa.ldq = ldq;
-  aa.ws = ctx->gemm_ws;
-  aa.ws_floats = kGemmWsFloats;
-  // fewer rows than kPrefillMinRows take the MFMA pass too where their
-  // operands are aligned for it
-  aa.mfma_ok = reinterpret_cast<uintptr_t>(aa.q) % 16 == 0 &&
-               reinterpret_cast<uintptr_t>(aa.out) % 16 == 0 && ldq % 4 == 0 &&
-               reinterpret_cast<uintptr_t>(aa.kc) % 16 == 0 &&
-               reinterpret_cast<uintptr_t>(aa.vc) % 16 == 0;
-  hipError_t e = q8::launch_attention(aa, ctx->stream);
+  hipError_t e;
+  if (s >= q8::kPrefillMinRows) {
+    aa.ws = ctx->gemm_ws;
+    aa.ws_floats = kGemmWsFloats;
+    e = with_scratch(ctx, [&] { return q8::launch_attention(aa, ctx->stream); });
+  } else {
+    // fewer rows take the MFMA pass too where their operands are aligned for
+    // it; the caller's scratch holds the records of a split per 64 keys
+    aa.ws = aa.part;
+    aa.ws_floats = (int64_t)sn;
+    aa.mfma_ok = reinterpret_cast<uintptr_t>(aa.q) % 16 == 0 &&
+                 reinterpret_cast<uintptr_t>(aa.out) % 16 == 0 && ldq % 4 == 0 &&
+                 reinterpret_cast<uintptr_t>(aa.part) % 16 == 0 &&
+                 reinterpret_cast<uintptr_t>(aa.kc) % 16 == 0 &&
+                 reinterpret_cast<uintptr_t>(aa.vc) % 16 == 0;
+    e = q8::launch_attention(aa, ctx->stream);
+  }
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_attention launch");
   return ok(ctx);
 }
@@ -1371,7 +1445,7 @@ int q8_decode_attention(q8_ctx *ctx, q8_buf *a, uint64_t oq_f32, uint64_t ok_f32
   da.posp = posbuf ? reinterpret_cast<const int *>(bytes(posbuf, opos_i32 * 4)) : nullptr;
   da.pos0 = (int)pos0;
   da.maxlen = (int)maxlen;
-  hipError_t e = q8::launch_decode_attention(da, ctx->stream);
+  hipError_t e = with_scratch(ctx, [&] { return q8::launch_decode_attention(da, ctx->stream); });
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_decode_attention launch");
   return ok(ctx);
 }
@@ -1509,7 +1583,8 @@ int q8_graph_begin(q8_ctx *ctx) {
   if (int rc = check_ctx(ctx)) return rc;
   if (ctx->host_only) return fail(ctx, Q8_ERR_NODEVICE, "q8_graph_begin: host-only context");
   if (int rc = set_device(ctx)) return rc;
-  hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
+  hipError_t e = mark_use(ctx);
+  if (e == hipSuccess) e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_graph_begin");
   return ok(ctx);
 }
@@ -1547,7 +1622,8 @@ int q8_graph_launch(q8_ctx *ctx, void *graph) {
   if (!graph) return fail(ctx, Q8_ERR_ARG, "q8_graph_launch: null graph");
   if (ctx->host_only) return fail(ctx, Q8_ERR_NODEVICE, "q8_graph_launch: host-only context");
   if (int rc = set_device(ctx)) return rc;
-  hipError_t e = hipGraphLaunch(static_cast<q8_graph *>(graph)->exec, ctx->stream);
+  hipError_t e = with_scratch(
+      ctx, [&] { return hipGraphLaunch(static_cast<q8_graph *>(graph)->exec, ctx->stream); });
   if (e != hipSuccess) return hip_fail(ctx, e, "q8_graph_launch");
   return ok(ctx);
 }

@@ -1059,3 +1059,102 @@ def test_token_begin_equals_uploads_and_gather(ctx, G, scale, d, token):
     assert list(pb.download((4,), np.int32)) == [77, 77, 1234, 77]
     for b in (w, a, ids, pb):
         b.free()
+
+
+def test_scratch_is_ordered_over_streams(ctx):
+    """Calls of one context on alternating streams, nothing else ordering
+    them: those that share the context's scratch (fragments, GEMM rows, split
+    records) run one behind the other, eagerly, after a graph's replay and
+    beside calls recorded into one, and leave the bits of calls on one
+    stream."""
+    import torch
+    say("scratch over streams")
+    rng = np.random.default_rng(3)
+    G, scale = 64, "f16"
+    runs = []                     # (call, arena, output offset, shape)
+
+    def linear(s, m, n, off):
+        pk = pack_q8_np(rng.standard_normal((n, m)).astype(np.float32), G, scale)
+        w = ctx.alloc(pk.nbytes + 2 * off)
+        w.upload(pk, 2 * off)
+        a = arena(ctx, s * m + s * n + 4)
+        put(a, 0, rng.standard_normal((s, m)).astype(np.float32))
+        oy = (s * m + 3) // 4 * 4
+        runs.append((lambda: q8hip.linear(ctx, w, off, a, 0, oy, s, m, n, G, scale), a, oy, (s, n)))
+
+    def attention(s, pos0, nh, nkv, hd):
+        n, kvd = pos0 + s, nkv * hd
+        kv = ctx.alloc(4 * n * kvd)
+        kv.upload(rng.standard_normal((2, n, kvd)).astype(np.float16))
+        a = arena(ctx, 2 * s * nh * hd)
+        put(a, 0, rng.standard_normal((s, nh * hd)).astype(np.float32))
+        oy = s * nh * hd
+        runs.append((lambda: q8hip.attention(ctx, a, 0, kv, 0, n * kvd, n, oy, 0, s, pos0, nh, nkv,
+                                             hd), a, oy, (s, nh * hd)))
+
+    linear(96, 4160, 1500, 3)
+    attention(33, 3000, 8, 2, 128)
+    linear(31, 4096, 2048, 0)
+    linear(64, 2048, 1024, 0)
+    attention(64, 2000, 16, 4, 64)
+    linear(20, 1600, 4000, 1)
+
+    def collect(call_all):
+        for _, a, oy, shape in runs:
+            put(a, oy, np.full(shape, np.nan, np.float32))
+        torch.cuda.synchronize()
+        call_all()
+        torch.cuda.synchronize()
+        return [get(a, oy, shape) for _, a, oy, shape in runs]
+
+    want = collect(lambda: [r[0]() for r in runs])
+    ctx.graph_begin()
+    try:
+        runs[0][0]()
+        runs[1][0]()
+    finally:
+        g = ctx.graph_end()
+    streams = [torch.cuda.Stream().cuda_stream, None, torch.cuda.Stream().cuda_stream]
+
+    def alternate():
+        for rep in range(6):
+            for k, r in enumerate(runs):
+                ctx.set_stream(streams[(rep + k) % 3])
+                r[0]()
+
+    def replay():
+        for rep in range(6):
+            for k, st in enumerate(streams):
+                ctx.set_stream(st)
+                g.launch()
+                ctx.set_stream(streams[(k + rep) % 3])
+                for r in runs[2:]:
+                    r[0]()
+
+    def beside_a_capture():
+        ctx.set_stream(streams[0])
+        runs[0][0]()
+        ctx.set_stream(None)
+        ctx.graph_begin()
+        try:
+            runs[0][0]()
+            runs[4][0]()
+        finally:
+            g2 = ctx.graph_end()
+        ctx.set_stream(streams[2])
+        for r in runs[1:]:
+            r[0]()
+        ctx.set_stream(None)
+        g2.launch()
+        ctx.sync()
+        g2.destroy()
+
+    try:
+        for how in (alternate, replay, beside_a_capture):
+            got = collect(how)
+            for k, (y, ref) in enumerate(zip(got, want)):
+                assert np.array_equal(y, ref), (how.__name__, k)
+    finally:
+        ctx.set_stream(None)
+        ctx.sync()
+        g.destroy()
