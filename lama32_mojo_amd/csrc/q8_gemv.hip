@@ -17,7 +17,7 @@
 //     arrival (the loop over a chunk has no branch, see compute_chunk);
 //   * the lane's 16 codes lie inside one quantization group (16 | G), so one
 //     scale per row per step is applied after the unscaled 16-term dot;
-//   * x (S rows of m f32) is staged once per workgroup in LDS and read with
+//   * x (m f32) is staged once per workgroup in LDS and read with
 //     ds_read_b128, or held in registers (a wave K range of at most 2
 //     steps); either way its loads are issued before the weights;
 //   * each (row, batch) partial is reduced across the wave with DPP row
@@ -68,21 +68,21 @@ __device__ __forceinline__ f32x4 load_f4(const float *p) {
   else return *reinterpret_cast<const f32x4 *>(p);
 }
 
-template <int G, int KIND, int S, int R, int SPLITK, bool XLDS, int PRE = PRE_NONE,
+template <int G, int KIND, int R, int SPLITK, bool XLDS, int PRE = PRE_NONE,
           int POST = POST_STORE, int NPF = 1, int NW = kWaves, bool UA = false>
 __global__ __launch_bounds__(64 * NW) void gemv_kernel(
     const uint8_t *__restrict__ w, int64_t row_bytes, int64_t n,
     const float *__restrict__ x, int64_t m, float *y, const uint16_t *__restrict__ wn,
     float eps, const float *res, float *__restrict__ amax) {
   extern __shared__ float xs[];
-  __shared__ float part[SPLITK > 1 ? NW : 1][R][S];
+  __shared__ float part[SPLITK > 1 ? NW : 1][R];
   __shared__ float red[4];
   static_assert(NW == kWaves || (SPLITK > 1 && NW % SPLITK == 0 && PRE != PRE_RMSNORM),
                 "workgroups of more than 4 waves are K-split row groups (no rmsnorm prologue)");
-  static_assert(PRE == PRE_NONE || (XLDS && S == 1), "fused prologues stage one x row in LDS");
-  static_assert(POST != POST_SWIGLU || (SPLITK == 1 && R % 2 == 0 && S == 1),
+  static_assert(PRE == PRE_NONE || XLDS, "fused prologues stage x in LDS");
+  static_assert(POST != POST_SWIGLU || (SPLITK == 1 && R % 2 == 0),
                 "the swiglu epilogue pairs gate and up rows within a wave");
-  static_assert(POST != POST_ARGMAX || (SPLITK == 1 && S == 1),
+  static_assert(POST != POST_ARGMAX || SPLITK == 1,
                 "the argmax epilogue keeps whole rows per wave");
   constexpr int SB = ScaleTraits<KIND>::bytes;
   constexpr int NT = 64 * NW;                   // threads
@@ -147,21 +147,20 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
   for (int r = 0; r < R; ++r) rowp[r] = w + row_of(r0, r) * row_bytes;
 
   // Load order at the start: loads return in issue order, so x goes first
-  // (its first staging batch, or with x read from L2 and one activation row
-  // this lane's x slices of the first NPF <= 2 steps, held in registers),
+  // (its first staging batch, or with x read from L2 this lane's x slices of
+  // the first NPF <= 2 steps, held in registers),
   // then every weight step of the first tile.  Staging x then waits for x
   // alone while the weights are still arriving.
   constexpr int XB = 4;                          // staging batch: 16-byte loads per thread
-  constexpr bool XREG = !XLDS && S == 1 && NPF <= 2;
+  constexpr bool XREG = !XLDS && NPF <= 2;
   f32x4 xv[XB], uv[XB];
   uint2 wb[XB];
   f32x4 xr[XREG ? NPF : 1][4];
-  const int64_t tot = S * m;                     // multiple of 4 (m % 32 == 0)
   auto load_x = [&](int64_t i0) {
 #pragma unroll
     for (int u = 0; u < XB; ++u) {
       const int64_t i = i0 + 4 * NT * u;
-      if (i < tot) {
+      if (i < m) {                                // (m is a multiple of 4)
         xv[u] = load_f4<UA>(x + i);
         if constexpr (PRE == PRE_SWIGLU) uv[u] = *reinterpret_cast<const f32x4 *>(x + m + i);
         if constexpr (PRE == PRE_RMSNORM) wb[u] = *reinterpret_cast<const uint2 *>(wn + i);
@@ -182,27 +181,20 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
   // POST_RESIDUAL: the first tile's residual values, loaded after the
   // weights (the store at the end would otherwise wait on one more round
   // trip).  Without a K split lane 0 stores the wave's outputs, so every
-  // lane holds them all; with one, thread t < R S stores output (t / S,
-  // t % S).  Indices past the outputs are clamped (their stores are
-  // skipped).  A residual that is y itself is read before this kernel
-  // writes any of it.
-  constexpr int RR = POST == POST_RESIDUAL ? (SPLITK > 1 ? 1 : RO * S) : 1;
+  // lane holds them all; with one, thread t < R stores output t.  Indices
+  // past the outputs are clamped (their stores are skipped).  A residual
+  // that is y itself is read before this kernel writes any of it.
+  constexpr int RR = POST == POST_RESIDUAL ? (SPLITK > 1 ? 1 : RO) : 1;
   float resv[RR] = {};
   if constexpr (POST == POST_RESIDUAL) {
     if constexpr (SPLITK > 1) {
-      // thread t < RG R S: row group t / (R S), row (t / S) % R, batch t % S
-      const int t = threadIdx.x < RG * R * S ? threadIdx.x : 0;
-      const int64_t tr = r0 - rgw * RO + (t / (R * S)) * RO + (t / S) % R;
-      const int64_t o = tr < nout ? tr : nout - 1;
-      resv[0] = res[(t % S) * n + o];
+      // thread t < RG R: row group t / R, row t % R
+      const int t = threadIdx.x < RG * R ? threadIdx.x : 0;
+      const int64_t tr = r0 - rgw * RO + (t / R) * RO + t % R;
+      resv[0] = res[tr < nout ? tr : nout - 1];
     } else {
 #pragma unroll
-      for (int r = 0; r < RO; ++r)
-#pragma unroll
-        for (int b = 0; b < S; ++b) {
-          const int64_t o = r0 + r < nout ? r0 + r : nout - 1;
-          resv[r * S + b] = res[b * n + o];
-        }
+      for (int r = 0; r < RO; ++r) resv[r] = res[r0 + r < nout ? r0 + r : nout - 1];
     }
   }
   // Every load above stays ahead of the first use: without this the
@@ -219,12 +211,12 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
     float ss = 0.0f;
     // batches of XB independent 16-byte loads per thread, then the LDS
     // stores (a load-store-load chain would wait on L2 once per step)
-    for (int64_t i0 = 4 * threadIdx.x; i0 < tot; i0 += 4 * NT * XB) {
+    for (int64_t i0 = 4 * threadIdx.x; i0 < m; i0 += 4 * NT * XB) {
       if (i0 != 4 * threadIdx.x) load_x(i0);     // the first batch is in flight already
 #pragma unroll
       for (int u = 0; u < XB; ++u) {
         const int64_t i = i0 + 4 * NT * u;
-        if (i >= tot) continue;
+        if (i >= m) continue;
         f32x4 o = xv[u];
         if constexpr (PRE == PRE_SWIGLU) {
           // x holds [gate | up]: 2m floats
@@ -259,7 +251,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
 
   // one finished output (value v of tile slot r) -> memory
   // (rv: the prefetched residual, used for the first tile)
-  auto store = [&](int64_t t0, int r, int b, float v, float v_up, float rv, bool first_tile) {
+  auto store = [&](int64_t t0, int r, float v, float v_up, float rv, bool first_tile) {
     const int64_t o = t0 + r;
     if (o >= nout) return;
     if constexpr (POST == POST_SWIGLU) {
@@ -267,8 +259,8 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
       y[o] = (g / (1.0f + expf(-g))) * u;
     } else {
       v = inv * v;
-      if constexpr (POST == POST_RESIDUAL) v = (first_tile ? rv : res[b * n + o]) + v;
-      y[b * n + o] = v;
+      if constexpr (POST == POST_RESIDUAL) v = (first_tile ? rv : res[o]) + v;
+      y[o] = v;
     }
   };
 
@@ -284,60 +276,53 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
   // every wave wait for all of its loads, and with x read from L2 inside
   // it, for one more round trip per step).
   const int64_t kx_safe = k_first < k_hi ? k_first : k_lo;
-  auto compute_chunk = [&](int64_t kw, float (&acc)[R][S]) {
+  auto compute_chunk = [&](int64_t kw, float (&acc)[R]) {
     const int64_t kc = kw + 16 * lane;
 #pragma unroll
     for (int p = 0; p < NPF; ++p) {
       const int64_t k = kc + 1024 * p;
       const bool live = k < k_hi;
       const int64_t kx = live ? k : kx_safe;
+      f32x4 xa, xb, xc, xd;
+      if (XREG && kw == k_lo) {
+        xa = xr[XREG ? p : 0][0];
+        xb = xr[XREG ? p : 0][1];
+        xc = xr[XREG ? p : 0][2];
+        xd = xr[XREG ? p : 0][3];
+      } else {
+        // (staged x is aligned whatever the call's x is)
+        const float *xq = xp + (XPAD ? xs_index(kx) : kx);
+        xa = load_f4<UA && !XLDS>(xq);
+        xb = load_f4<UA && !XLDS>(xq + 4);
+        xc = load_f4<UA && !XLDS>(xq + 8);
+        xd = load_f4<UA && !XLDS>(xq + 12);
+      }
 #pragma unroll
-      for (int b = 0; b < S; ++b) {
-        f32x4 xa, xb, xc, xd;
-        if (XREG && kw == k_lo) {
-          xa = xr[XREG ? p : 0][0];
-          xb = xr[XREG ? p : 0][1];
-          xc = xr[XREG ? p : 0][2];
-          xd = xr[XREG ? p : 0][3];
-        } else {
-          // (staged x is aligned whatever the call's x is)
-          const float *xq = xp + (XPAD ? xs_index(b * m + kx) : b * m + kx);
-          xa = load_f4<UA && !XLDS>(xq);
-          xb = load_f4<UA && !XLDS>(xq + 4);
-          xc = load_f4<UA && !XLDS>(xq + 8);
-          xd = load_f4<UA && !XLDS>(xq + 12);
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const float t = __builtin_fmaf(sc[p][r], dot16(q[p][r], xa, xb, xc, xd), acc[r][b]);
-          acc[r][b] = live ? t : acc[r][b];
-        }
+      for (int r = 0; r < R; ++r) {
+        const float t = __builtin_fmaf(sc[p][r], dot16(q[p][r], xa, xb, xc, xd), acc[r]);
+        acc[r] = live ? t : acc[r];
       }
     }
   };
 
   // A finished tile: wave sums, the K split's partials met in LDS, the
   // epilogue.
-  auto finish_tile = [&](int64_t t0, const float (&acc)[R][S], bool first_tile) {
+  auto finish_tile = [&](int64_t t0, const float (&acc)[R], bool first_tile) {
     if constexpr (SPLITK == 1) {
-      float v[R][S];
+      float v[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int b = 0; b < S; ++b) v[r][b] = wave_sum(acc[r][b]);
+      for (int r = 0; r < R; ++r) v[r] = wave_sum(acc[r]);
       if (lane == 0) {
 #pragma unroll
         for (int r = 0; r < RO; ++r)
-#pragma unroll
-          for (int b = 0; b < S; ++b)
-            store(t0, r, b, v[r][b], POST == POST_SWIGLU ? v[(r + RO) % R][b] : 0.0f,
-                  resv[POST == POST_RESIDUAL ? r * S + b : 0], first_tile);
+          store(t0, r, v[r], POST == POST_SWIGLU ? v[(r + RO) % R] : 0.0f,
+                resv[POST == POST_RESIDUAL ? r : 0], first_tile);
         if constexpr (POST == POST_ARGMAX) {
           // rows in increasing order, strict >: the lowest row among equal
           // values; NaN never wins
 #pragma unroll
           for (int r = 0; r < R; ++r) {
-            const float yv = inv * v[r][0];
+            const float yv = inv * v[r];
             if (t0 + r < n && yv > best_v) {
               best_v = yv;
               best_i = (int)(t0 + r);
@@ -347,19 +332,17 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
       }
     } else {
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int b = 0; b < S; ++b) {
-          float v = wave_sum(acc[r][b]);
-          if (lane == 0) part[wid][r][b] = v;
-        }
+      for (int r = 0; r < R; ++r) {
+        const float v = wave_sum(acc[r]);
+        if (lane == 0) part[wid][r] = v;
+      }
       __syncthreads();
-      if (threadIdx.x < RG * R * S) {
-        const int g = threadIdx.x / (R * S), r = (threadIdx.x / S) % R, b = threadIdx.x % S;
-        float v = part[g * SPLITK][r][b];
+      if (threadIdx.x < RG * R) {
+        const int g = threadIdx.x / R, r = threadIdx.x % R;
+        float v = part[g * SPLITK][r];
 #pragma unroll
-        for (int u = 1; u < SPLITK; ++u) v += part[g * SPLITK + u][r][b];
-        store(t0 - rgw * RO + g * RO, r, b, v, 0.0f, resv[0], first_tile);
+        for (int u = 1; u < SPLITK; ++u) v += part[g * SPLITK + u][r];
+        store(t0 - rgw * RO + g * RO, r, v, 0.0f, resv[0], first_tile);
       }
       __syncthreads();
     }
@@ -371,11 +354,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
   // the clamped rows it loaded and stores nothing), and every wave reaches
   // the barriers of finish_tile.
   {
-    float acc[R][S];
+    float acc[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int b = 0; b < S; ++b) acc[r][b] = 0.0f;
+    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
     compute_chunk(k_lo, acc);
     for (int64_t kw = k_lo + 1024 * NPF; kw < k_hi; kw += 1024 * NPF) {
       load_chunk(rowp, kw + 16 * lane);
@@ -386,11 +367,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
   for (r0 += stride_rows; r0 < nout; r0 += stride_rows) {
 #pragma unroll
     for (int r = 0; r < R; ++r) rowp[r] = w + row_of(r0, r) * row_bytes;
-    float acc[R][S];
+    float acc[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int b = 0; b < S; ++b) acc[r][b] = 0.0f;
+    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
     for (int64_t kw = k_lo; kw < k_hi; kw += 1024 * NPF) {
       load_chunk(rowp, kw + 16 * lane);
       compute_chunk(kw, acc);
@@ -479,11 +458,11 @@ hipError_t launch_fast_t(const LinearArgs &a, const float *x, float *y, int64_t 
   const bool xreg = NW == kWaves && NPF <= 2 && a.m / SPLITK <= 1024 * NPF;
   if ((NW > kWaves || a.m <= kLdsStageFloats) && !xreg) {
     size_t lds = (size_t)a.m * sizeof(float);
-    hipLaunchKernelGGL((gemv_kernel<G, KIND, 1, R, SPLITK, true, PRE_NONE, POST_STORE, NPF, NW, UA>),
+    hipLaunchKernelGGL((gemv_kernel<G, KIND, R, SPLITK, true, PRE_NONE, POST_STORE, NPF, NW, UA>),
                        grid, block, lds, st, a.w, a.row_bytes, a.n, x, a.m, y, nullptr, 0.0f,
                        nullptr, nullptr);
   } else if constexpr (NW == kWaves) {
-    hipLaunchKernelGGL((gemv_kernel<G, KIND, 1, R, SPLITK, false, PRE_NONE, POST_STORE, NPF, NW, UA>),
+    hipLaunchKernelGGL((gemv_kernel<G, KIND, R, SPLITK, false, PRE_NONE, POST_STORE, NPF, NW, UA>),
                        grid, block, 0, st, a.w, a.row_bytes, a.n, x, a.m, y, nullptr, 0.0f,
                        nullptr, nullptr);
   }
@@ -582,12 +561,12 @@ hipError_t launch_fused_npf(const FusedLinearArgs &f, int64_t cap, hipStream_t s
   if (f.grid_out) *f.grid_out = (int)grid.x;
   if constexpr (PRE == PRE_NONE && NW == kWaves) {
     if (a.m > kLdsStageFloats || (NPF <= 2 && a.m / SPLITK <= 1024 * NPF)) {
-      hipLaunchKernelGGL((gemv_kernel<G, KIND, 1, R, SPLITK, false, PRE, POST, NPF>), grid, block,
+      hipLaunchKernelGGL((gemv_kernel<G, KIND, R, SPLITK, false, PRE, POST, NPF>), grid, block,
                          0, st, a.w, a.row_bytes, a.n, x, a.m, a.y, f.wn, f.eps, f.res, f.part);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((gemv_kernel<G, KIND, 1, R, SPLITK, true, PRE, POST, NPF, NW>), grid, block,
+  hipLaunchKernelGGL((gemv_kernel<G, KIND, R, SPLITK, true, PRE, POST, NPF, NW>), grid, block,
                      (size_t)(x_padded(PRE, POST) ? xs_floats(a.m) : a.m) * sizeof(float), st,
                      a.w, a.row_bytes, a.n, x, a.m, a.y, f.wn,
                      f.eps, f.res, f.part);

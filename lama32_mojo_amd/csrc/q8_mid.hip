@@ -25,8 +25,8 @@
 // aligned rows of 4096 codes or more (31 x 4096 x 24576 65 -> 44 us; the line
 // is drawn in the dispatch).
 //
-// Layout: a workgroup owns 32 RT rows x 32 C KW columns, wave w 32 C
-// columns of them, and a range of 64-code units of K.  Per phase of PU units
+// Layout: a workgroup owns 32 RT rows x 32 KW columns, wave w 32 columns of
+// them, and a range of 64-code units of K.  Per phase of two units (PU)
 // the workgroup stages the tile's x fragments in LDS (double-buffered, one
 // barrier per phase) and each wave its own codes: loaded LPR lanes to a row,
 // in runs of 64 PU bytes, and read back from LDS as the MFMA takes them, 16
@@ -63,6 +63,7 @@ __device__ __forceinline__ u32x4 load_codes16(const uint8_t *p) {
 }
 
 constexpr int kUnit = 64;            // codes of a row per unit
+constexpr int PU = 2;                // units per phase
 // Workgroups that the K split aims at, one per CU: 512 made 16 x 4096 x
 // 28672 41.8 -> 44.0 us and 200 x 1600 x 4800 28.2 -> 35.8 us.
 constexpr int kTarget = 256;
@@ -203,9 +204,9 @@ __device__ __forceinline__ f16x8 codes_to_f16(uint32_t d0, uint32_t d1) {
 
 template <int N> struct __attribute__((packed, aligned(2))) Dwords { uint32_t d[N]; };
 
-// One workgroup: 32 RT rows x 32 C KW columns over units [u0, u1) of K, wave
-// w owning columns 32 C w .. of the tile.
-template <int G, int KIND, int NT, int RT, int C, int KW, int PU>
+// One workgroup: 32 RT rows x 32 KW columns over units [u0, u1) of K, wave
+// w owning columns 32 w .. of the tile.
+template <int G, int KIND, int NT, int RT, int KW>
 __global__ __launch_bounds__(64 * KW) __attribute__((amdgpu_waves_per_eu(2)))
 void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16 *__restrict__ xf,
                 const int *__restrict__ ex, float *__restrict__ y, int s, int m, int64_t n,
@@ -223,7 +224,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
   static_assert(XF % KW == 0 && PU * UB % 4 == 0, "whole fragments and scale dwords");
   __shared__ f16x8 xs[2][XF][64];
   __shared__ __attribute__((aligned(16))) int exs[32 * RT];
-  __shared__ __attribute__((aligned(16))) uint8_t cl[KW][32 * C][PU * kUnit + 16];
+  __shared__ __attribute__((aligned(16))) uint8_t cl[KW][32][PU * kUnit + 16];
 
   // Workgroups go to the 8 XCDs in turn: workgroup id runs on XCD id % 8.
   // The row blocks of a (column block, K split) take consecutive turns of
@@ -234,7 +235,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
   if (cb >= ncb) return;
   const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t n0 = ((int64_t)cb * KW + wid) * (32 * C);
+  const int64_t n0 = ((int64_t)cb * KW + wid) * 32;
   const int nu = (m + kUnit - 1) / kUnit;
   const int u0 = ks * upk;                             // (no split is empty)
   const int u1 = u0 + upk < nu ? u0 + upk : nu;
@@ -249,16 +250,13 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
   // are not stored.
   const int64_t nb = n0 < n ? n0 : n - 1;
   const uint8_t *wb = w + nb * row_bytes;
-  const int last = (int)(n - 1 - nb < 32 * C ? n - 1 - nb : 32 * C - 1);
+  const int last = (int)(n - 1 - nb < 32 ? n - 1 - nb : 31);
   const int piece = lane % LPR;
-  uint32_t coff[C][WL], soff[C];
+  const uint32_t soff = (uint32_t)(min(lr, last) * row_bytes);
+  uint32_t coff[WL];
 #pragma unroll
-  for (int c = 0; c < C; ++c) {
-    soff[c] = (uint32_t)(min(32 * c + lr, last) * row_bytes);
-#pragma unroll
-    for (int i = 0; i < WL; ++i)
-      coff[c][i] = (uint32_t)(min(32 * c + i * RPI + lane / LPR, last) * row_bytes + (m / G) * SB);
-  }
+  for (int i = 0; i < WL; ++i)
+    coff[i] = (uint32_t)(min(i * RPI + lane / LPR, last) * row_bytes + (m / G) * SB);
   // the fragments this wave stages: numbers wid + KW i of the phase's XF
   // (unit, row tile, fragment)
   const int ntile = (s + 31) / 32;
@@ -273,9 +271,9 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
   }
 
   const uint32_t lane16 = 16u * lane;
-  u32x4 W[2][C][WL];
+  u32x4 W[2][WL];
   f16x8 X[2][XL];
-  Dwords<SD> SC[2][C];
+  Dwords<SD> SC[2];
   // Units past u1 take the unit of zeros behind the row of x and reread the
   // codes of the last unit, and a last unit of 32 codes reads its first
   // piece twice: no load leaves its row.  (A scale load that starts in
@@ -292,15 +290,11 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
           reinterpret_cast<const uint8_t *>(xt[i] + (int64_t)u * (XU * 512)) + (lane16 & on));
     }
     const int us = up < u1 ? up : u1 - 1;
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-      SC[st][c] = *reinterpret_cast<const Dwords<SD> *>(wb + ((soff[c] + (uint32_t)(us * UB)) & on));
+    SC[st] = *reinterpret_cast<const Dwords<SD> *>(wb + ((soff + (uint32_t)(us * UB)) & on));
     const int un = up + piece / 4 < u1 ? up + piece / 4 : u1 - 1;
     const int k = un * kUnit + 16 * (un * kUnit + 32 < m ? piece & 3 : piece & 1);
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-      for (int i = 0; i < WL; ++i) W[st][c][i] = load_codes16(wb + ((coff[c][i] + (uint32_t)k) & on));
+    for (int i = 0; i < WL; ++i) W[st][i] = load_codes16(wb + ((coff[i] + (uint32_t)k) & on));
     __builtin_amdgcn_sched_barrier(0);
   };
   // register stage st to x buffer st and the wave's code rows (a wave's LDS
@@ -309,44 +303,38 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
 #pragma unroll
     for (int i = 0; i < XL; ++i) xs[st][wid + KW * i][lane] = X[st][i];
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-      for (int i = 0; i < WL; ++i)
-        *reinterpret_cast<u32x4 *>(&cl[wid][32 * c + i * RPI + lane / LPR][16 * piece]) = W[st][c][i];
+    for (int i = 0; i < WL; ++i)
+      *reinterpret_cast<u32x4 *>(&cl[wid][i * RPI + lane / LPR][16 * piece]) = W[st][i];
   };
 
-  f32x16 acc[RT][C];
+  f32x16 acc[RT];
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[t][c][v] = 0.0f;
+    for (int v = 0; v < 16; ++v) acc[t][v] = 0.0f;
 
   // The PU RT blocks (unit up + v, row tile t) of a phase, from register
   // stage and x buffer st.  A block's fragments are read from LDS one block
   // ahead, and its partials are folded into the output behind the MFMAs of
   // the next block.  Nothing is skipped: units past u1 and groups past m met
   // zeros of x, and their scale is forced to 0.
-  auto compute = [&](int st, int up, const Dwords<SD> (&scd)[C]) {
+  auto compute = [&](int st, int up, const Dwords<SD> &scd) {
     constexpr int NB = PU * RT;
-    f16x8 a[2][XU], b[C][4];
-    u32x4 q[2][C][2];
+    f16x8 a[2][XU], b[4];
+    u32x4 q[2][2];
     // (two groups per unit: their partials already fill the registers that
     // a second set would take)
     constexpr int DB = GPU_ == 1 ? 2 : 1;
-    f32x16 d[DB][C][GPU_];
+    f32x16 d[DB][GPU_];
     auto read_a = [&](int blk) {
 #pragma unroll
       for (int i = 0; i < XU; ++i) a[blk & 1][i] = xs[st][blk * XU + i][lane];
       if (blk % RT == 0) {
         const int v = blk / RT;
 #pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-          for (int p = 0; p < 2; ++p)
-            q[v & 1][c][p] = *reinterpret_cast<const u32x4 *>(
-                &cl[wid][32 * c + lr][kUnit * v + (G == 64 ? 32 * lh + 16 * p : 32 * p + 16 * lh)]);
+        for (int p = 0; p < 2; ++p)
+          q[v & 1][p] = *reinterpret_cast<const u32x4 *>(
+              &cl[wid][lr][kUnit * v + (G == 64 ? 32 * lh + 16 * p : 32 * p + 16 * lh)]);
       }
     };
     auto fold = [&](int blk) {
@@ -354,17 +342,13 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
 #pragma unroll
       for (int g = 0; g < GPU_; ++g) {
         const bool live = up + v < u1 && (up + v) * kUnit + g * G < m;
+        const int byte = v * UB + g * SB;
+        const uint32_t raw = scd.d[byte >> 2];
+        float sc = KIND == SCALE_F16 ? f16_bits_to_f32((uint16_t)(raw >> (8 * (byte & 3))))
+                                     : __builtin_bit_cast(float, raw);
+        sc = live ? sc : 0.0f;
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-          const int byte = v * UB + g * SB;
-          const uint32_t raw = scd[c].d[byte >> 2];
-          float sc = KIND == SCALE_F16 ? f16_bits_to_f32((uint16_t)(raw >> (8 * (byte & 3))))
-                                       : __builtin_bit_cast(float, raw);
-          sc = live ? sc : 0.0f;
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            acc[t][c][e] = __builtin_fmaf(sc, d[blk % DB][c][g][e], acc[t][c][e]);
-        }
+        for (int e = 0; e < 16; ++e) acc[t][e] = __builtin_fmaf(sc, d[blk % DB][g][e], acc[t][e]);
       }
     };
     read_a(0);
@@ -375,29 +359,25 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
       __builtin_amdgcn_sched_barrier(0);
       if (blk % RT == 0) {                     // the unit's codes, step 2 p + e
 #pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            b[c][2 * p] = codes_to_f16(q[v & 1][c][p].x, q[v & 1][c][p].y);
-            b[c][2 * p + 1] = codes_to_f16(q[v & 1][c][p].z, q[v & 1][c][p].w);
-          }
+        for (int p = 0; p < 2; ++p) {
+          b[2 * p] = codes_to_f16(q[v & 1][p].x, q[v & 1][p].y);
+          b[2 * p + 1] = codes_to_f16(q[v & 1][p].z, q[v & 1][p].w);
+        }
       }
 #pragma unroll
       for (int i = 0; i < SPG; ++i)
 #pragma unroll
         for (int term = 0; term < NT; ++term)
 #pragma unroll
-          for (int g = 0; g < GPU_; ++g)
+          for (int g = 0; g < GPU_; ++g) {
+            f32x16 z;
 #pragma unroll
-            for (int c = 0; c < C; ++c) {
-              f32x16 z;
-#pragma unroll
-              for (int e = 0; e < 16; ++e) z[e] = 0.0f;
-              const int step = g * SPG + i;
-              d[blk % DB][c][g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                  a[blk & 1][step * NT + term], b[c][step],
-                  i == 0 && term == 0 ? z : d[blk % DB][c][g], 0, 0, 0);
-            }
+            for (int e = 0; e < 16; ++e) z[e] = 0.0f;
+            const int step = g * SPG + i;
+            d[blk % DB][g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                a[blk & 1][step * NT + term], b[step],
+                i == 0 && term == 0 ? z : d[blk % DB][g], 0, 0, 0);
+          }
       if (DB == 1) fold(blk);
       if (DB == 2 && blk > 0) fold(blk - 1);
     }
@@ -418,9 +398,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
   do {
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
-      Dwords<SD> scd[C];
-#pragma unroll
-      for (int c = 0; c < C; ++c) scd[c] = SC[st][c];
+      const Dwords<SD> scd = SC[st];
       load_phase(st, up + 2 * PU);
       compute(st, up, scd);
       store_phase(st ^ 1);
@@ -440,21 +418,18 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
       typedef int i32x4 __attribute__((ext_vector_type(4)));
       const i32x4 e = *reinterpret_cast<const i32x4 *>(&exs[t * 32 + 8 * b + 4 * lh]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-          const int64_t j = n0 + 32 * c + lr;
-          const int r = r0 + 8 * b + i;
-          if (r < s && j < n)
-            out[(int64_t)r * n + j] = __builtin_ldexpf(acc[t][c][4 * b + i], e[i]);
-        }
+      for (int i = 0; i < 4; ++i) {
+        const int64_t j = n0 + lr;
+        const int r = r0 + 8 * b + i;
+        if (r < s && j < n) out[(int64_t)r * n + j] = __builtin_ldexpf(acc[t][4 * b + i], e[i]);
+      }
     }
   }
 }
 
-template <int G, int KIND, int NT, int RT, int C, int KW, int PU>
+template <int G, int KIND, int NT, int RT, int KW>
 hipError_t launch_t(const LinearArgs &a, const _Float16 *xf, const int *ex, hipStream_t st) {
-  const int64_t ncb = (a.n + 32 * C * KW - 1) / (32 * C * KW), nrb = (a.s + 32 * RT - 1) / (32 * RT);
+  const int64_t ncb = (a.n + 32 * KW - 1) / (32 * KW), nrb = (a.s + 32 * RT - 1) / (32 * RT);
   const int nu = (int)((a.m + kUnit - 1) / kUnit);
   int nks = 1;
   if (a.ws)
@@ -464,7 +439,7 @@ hipError_t launch_t(const LinearArgs &a, const _Float16 *xf, const int *ex, hipS
   const int upk = ((nu + nks - 1) / nks + 2 * PU - 1) / (2 * PU) * (2 * PU);
   nks = (nu + upk - 1) / upk;                          // no empty split
   const int64_t blocks = (ncb * nks + 7) / 8 * 8 * nrb;
-  hipLaunchKernelGGL((mid_kernel<G, KIND, NT, RT, C, KW, PU>), dim3((unsigned)blocks), dim3(64 * KW),
+  hipLaunchKernelGGL((mid_kernel<G, KIND, NT, RT, KW>), dim3((unsigned)blocks), dim3(64 * KW),
                      0, st, a.w, a.row_bytes, xf, ex, a.y, (int)a.s, (int)a.m, a.n, (int)ncb,
                      (int)nrb, nks, upk, a.ws);
   if (nks > 1) return launch_splitk_reduce(a.ws, a.y, a.s * a.n, nks, st);
@@ -475,12 +450,12 @@ template <int G, int KIND>
 hipError_t launch_g(const LinearArgs &a, _Float16 *xf, int *ex, hipStream_t st) {
   if (a.x_is_bf16) {
     launch_frag16<false, 1, G>(a, xf, ex, st);
-    if (a.s <= 32) return launch_t<G, KIND, 1, 1, 1, 4, 2>(a, xf, ex, st);
-    return launch_t<G, KIND, 1, 2, 1, 8, 2>(a, xf, ex, st);
+    if (a.s <= 32) return launch_t<G, KIND, 1, 1, 4>(a, xf, ex, st);
+    return launch_t<G, KIND, 1, 2, 8>(a, xf, ex, st);
   }
   launch_frag16<true, 2, G>(a, xf, ex, st);
-  if (a.s <= 32) return launch_t<G, KIND, 2, 1, 1, 4, 2>(a, xf, ex, st);
-  return launch_t<G, KIND, 2, 2, 1, 8, 2>(a, xf, ex, st);
+  if (a.s <= 32) return launch_t<G, KIND, 2, 1, 4>(a, xf, ex, st);
+  return launch_t<G, KIND, 2, 2, 8>(a, xf, ex, st);
 }
 
 }  // namespace
