@@ -99,7 +99,7 @@ hipError_t launch_skinny(const LinearArgs &a, hipStream_t st);
 constexpr int kSkinny4MaxRows = 4;
 hipError_t launch_skinny4(const LinearArgs &a, hipStream_t st);
 
-// Any alignment, f32 or bf16 x: binary16 fragments of x in `bytes` of scratch
+// Any alignment, f32 or bf16 x: bf16 fragments of x in `bytes` of scratch
 // (16-byte aligned), then MFMA on the codes as read; in chunks of as many rows as
 // mid_rows gives (0: a row tile does not fit, hipErrorInvalidValue).
 int64_t mid_rows(int64_t bytes, int64_t m, bool x_is_bf16);

@@ -5,24 +5,28 @@
 // (k_mm_q8, src/llama_q8.mojo:54-93: unscaled dot per group, then one scale
 // multiply per group), in two launches (a third, splitk_reduce_kernel, adds
 // the partial sums when K is split over workgroups):
-//   1. frag16_kernel writes x as binary16 MFMA fragments.  Each row is
-//      scaled by a power of two so that its largest finite |x| lies in
-//      [2^14, 2^15); with NT = 2 (f32 x) it is split into hi = f16(x) and
-//      lo = f16(x - hi), which carries x to 2^-22 (and to 2^-39 of the row's
-//      largest value below binary16's normal range); with NT = 1 (bf16 x) hi
-//      alone is exact;
-//   2. mid_kernel runs v_mfma_f32_32x32x16_f16 on the fragments and the
-//      codes.  |q| <= 127 is exact in binary16, so the products are exact;
+//   1. frag_kernel writes x as bf16 MFMA fragments: bf16 x as it is (NT = 1),
+//      f32 x cut into NT = 3 terms of 8 bits each, whose sum is x.  (Each row
+//      is scaled by a power of two so that its largest finite |x| lies in
+//      [2^14, 2^15), which keeps the terms of the smallest rows in bf16's
+//      range: what they leave out lies below 2^-140 of the row's largest
+//      value.)
+//   2. mid_kernel runs v_mfma_f32_32x32x16_bf16 on the fragments and the
+//      codes.  |q| <= 127 is exact in bf16, so the products are exact;
 //      a group's partial starts from 0 and is folded into the output with
 //      one f32 FMA by the group's scale, as the reference does.
-// Its error is that of the f32 sums (about 1e-7 of float64).
+// Its error is that of the f32 sums (about 1e-7 of float64).  Two binary16
+// terms of a scaled row take two MFMAs instead of three and are 10-30 %
+// faster at the same error on ordinary rows (200 x 1600 x 4800 28 us against
+// 32, 512 x 11008 x 4096 127 against 166), but carry x to 2^-39 of its row's
+// largest value only: beside a channel of 2^34 the rest lost percents.
 //
 // Where it runs: rows or x that are not 16-byte aligned (a row is (m / G) SB
 // + m bytes, so most widths that are no multiple of 512 at G = 64 with f16
 // scales), against one wave per output with one code per lane and load:
-// 200 x 1600 x 4800 1030 -> 28 us, 512 x 11008 x 4096 24390 -> 133 us, 16 x
-// 11008 x 4096 777 -> 24 us, 2 x 1600 x 4800 17 -> 12.5 us; and 17 .. 31
-// aligned rows of 4096 codes or more (31 x 4096 x 24576 65 -> 44 us; the line
+// 200 x 1600 x 4800 1030 -> 32 us, 512 x 11008 x 4096 24390 -> 166 us, 20 x
+// 11008 x 4096 970 -> 28 us; and 17 .. 31
+// aligned rows of 4096 codes or more (31 x 4096 x 24576 65 -> 45 us; the line
 // is drawn in the dispatch).
 //
 // Layout: a workgroup owns 32 RT rows x 32 KW columns, wave w 32 columns of
@@ -35,12 +39,13 @@
 // different rows: 16 x 4096 x 28672 took 45 us that way against 37.)
 // The order of k within a unit is free as long as a step stays in its
 // group: lane half h feeds codes 32 h + 16 p + 8 e .. +8 in step 2 p + e
-// (G = 64), or 32 p + 16 h + 8 e .. +8 (G = 32); frag16_kernel lays x out to
+// (G = 64), or 32 p + 16 h + 8 e .. +8 (G = 32); frag_kernel lays x out to
 // match, one contiguous KiB per (32 rows, step, term).
-// What bounds it: with 256 workgroups a phase of 2 units takes about 0.9 us
-// at RT = 1, 4.7 TB/s of codes; about 5 us per launch are its start, the
-// first loads and the last stores, and the two launches around it cost 3 us
-// each, which is what small shapes pay (16 x 1600 x 4800: 12.9 us).
+// What bounds it: below about 100 rows the codes' way through a phase of
+// two units (1.1 us at RT = 1 and 256 workgroups), then the MFMAs; about 5 us
+// per launch are its start, the first loads and the last stores, and the two
+// launches around it cost 3 us each, which is what small shapes pay (16 x
+// 1600 x 4800: 14 us).
 //
 // Alignment: packed rows start at any even byte, so codes and scales are
 // loaded as vectors of 2-byte alignment (one instruction; the hardware
@@ -51,8 +56,6 @@
 namespace q8 {
 namespace {
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 // 16 bytes at 2-byte (packed rows), 4-byte (f32 x) or 2-byte (bf16 x) alignment
 struct __attribute__((packed, aligned(2))) Codes16 { uint32_t d[4]; };
 struct __attribute__((packed, aligned(4))) Floats4 { float v[4]; };
@@ -68,19 +71,19 @@ constexpr int PU = 2;                // units per phase
 // 28672 41.8 -> 44.0 us and 200 x 1600 x 4800 28.2 -> 35.8 us.
 constexpr int kTarget = 256;
 
-// ---- 1. x as binary16 fragments ---------------------------------------------
+// ---- 1. x as bf16 fragments ---------------------------------------------------
 // One 256-thread block per row r.  Fragment block (row tile r / 32, unit,
-// step, term) is 64 lanes x 8 halves; see the file comment for the order of
+// step, term) is 64 lanes x 8 values; see the file comment for the order of
 // k.  Values past m (a last unit of 32 codes, and one unit of zeros behind
 // the row) are zeros.  The exponent is
 // that of the largest finite value: infinities and NaN stay what they are in
-// hi (lo = 0) and do not change the rest of their row.
+// the first term (the others 0) and do not change the rest of their row.
 // With CH > 0 the row (m <= 2048 CH) stays in registers between the maximum
 // and the conversion; CH = 0 reads it twice.
 template <bool XF32, int NT, int G, int CH>
-__global__ __launch_bounds__(256) void frag16_kernel(const void *__restrict__ xv, int64_t m,
-                                                     _Float16 *__restrict__ xf,
-                                                     int *__restrict__ ex) {
+__global__ __launch_bounds__(256) void frag_kernel(const void *__restrict__ xv, int64_t m,
+                                                   __bf16 *__restrict__ xf,
+                                                   int *__restrict__ ex) {
   __shared__ float red[4];
   const int64_t r = blockIdx.x;
   const int tid = threadIdx.x;
@@ -140,23 +143,30 @@ __global__ __launch_bounds__(256) void frag16_kernel(const void *__restrict__ xv
     e = (int)((__builtin_bit_cast(uint32_t, mx) >> 23) & 255u) - 127 - 14;
     e = e < -126 ? -126 : e;                 // (subnormal maxima: as far as 2^126 goes)
   }
-  _Float16 *row = xf + (r >> 5) * (nu + 1) * (4 * NT * 512) + (r & 31) * 8;
+  __bf16 *row = xf + (r >> 5) * (nu + 1) * (4 * NT * 512) + (r & 31) * 8;
   auto store8 = [&](int64_t k, const float (&v)[8]) {
     const int kk = (int)(k & 63);
     const int hf = G == 64 ? kk >> 5 : (kk >> 4) & 1;
     const int p = G == 64 ? (kk >> 4) & 1 : kk >> 5;
     const int step = 2 * p + ((kk >> 3) & 1);
-    _Float16 *dst = row + ((k >> 6) * 4 + step) * (NT * 512) + hf * 256;
-    f16x8 hi, lo;
+    __bf16 *dst = row + ((k >> 6) * 4 + step) * (NT * 512) + hf * 256;
+    float rest[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float s = __builtin_ldexpf(v[j], -e);
-      hi[j] = (_Float16)s;
-      const float d = s - (float)hi[j];
-      lo[j] = (_Float16)(d == d ? d : 0.0f);   // inf - inf and NaN: hi alone
+    for (int j = 0; j < 8; ++j) rest[j] = __builtin_ldexpf(v[j], -e);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      // the upper 8 bits of what is left; the subtraction is exact
+      u32x4 o;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c] = pk_hi16(rest[2 * c], rest[2 * c + 1]);
+      *reinterpret_cast<u32x4 *>(dst + 512 * t) = o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float d = rest[j] - __builtin_bit_cast(
+            float, __builtin_bit_cast(uint32_t, rest[j]) & 0xffff0000u);
+        rest[j] = d == d ? d : 0.0f;           // inf - inf and NaN: the first term alone
+      }
     }
-    *reinterpret_cast<f16x8 *>(dst) = hi;
-    if constexpr (NT == 2) *reinterpret_cast<f16x8 *>(dst + 512) = lo;
   };
   const int64_t kend = (nu + 1) * kUnit;
   if constexpr (CH > 0) {
@@ -179,36 +189,24 @@ __global__ __launch_bounds__(256) void frag16_kernel(const void *__restrict__ xv
 }
 
 template <bool XF32, int NT, int G>
-void launch_frag16(const LinearArgs &a, _Float16 *xf, int *ex, hipStream_t st) {
+void launch_frag(const LinearArgs &a, __bf16 *xf, int *ex, hipStream_t st) {
   const dim3 grid((unsigned)a.s), block(256);
   if (a.m <= 4096)
-    hipLaunchKernelGGL((frag16_kernel<XF32, NT, G, 2>), grid, block, 0, st, a.x, a.m, xf, ex);
+    hipLaunchKernelGGL((frag_kernel<XF32, NT, G, 2>), grid, block, 0, st, a.x, a.m, xf, ex);
   else if (a.m <= 16384)
-    hipLaunchKernelGGL((frag16_kernel<XF32, NT, G, 8>), grid, block, 0, st, a.x, a.m, xf, ex);
+    hipLaunchKernelGGL((frag_kernel<XF32, NT, G, 8>), grid, block, 0, st, a.x, a.m, xf, ex);
   else
-    hipLaunchKernelGGL((frag16_kernel<XF32, NT, G, 0>), grid, block, 0, st, a.x, a.m, xf, ex);
+    hipLaunchKernelGGL((frag_kernel<XF32, NT, G, 0>), grid, block, 0, st, a.x, a.m, xf, ex);
 }
 
 // ---- 2. the linear ------------------------------------------------------------
-// Eight codes (two dwords, k order) as exact binary16.
-__device__ __forceinline__ f16x8 codes_to_f16(uint32_t d0, uint32_t d1) {
-  const f16x2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
-  const uint32_t x0 = d0 ^ 0x80808080u, x1 = d1 ^ 0x80808080u;   // q + 128 per byte
-  // binary16 0x64hh = 1024 + hh exactly; minus 1152 gives q exactly
-  const f16x2 a = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, x0, 0x04010400u)) - off;
-  const f16x2 b = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, x0, 0x04030402u)) - off;
-  const f16x2 c = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, x1, 0x04010400u)) - off;
-  const f16x2 d = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, x1, 0x04030402u)) - off;
-  return f16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-}
-
 template <int N> struct __attribute__((packed, aligned(2))) Dwords { uint32_t d[N]; };
 
 // One workgroup: 32 RT rows x 32 KW columns over units [u0, u1) of K, wave
 // w owning columns 32 w .. of the tile.
 template <int G, int KIND, int NT, int RT, int KW>
 __global__ __launch_bounds__(64 * KW) __attribute__((amdgpu_waves_per_eu(2)))
-void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16 *__restrict__ xf,
+void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const __bf16 *__restrict__ xf,
                 const int *__restrict__ ex, float *__restrict__ y, int s, int m, int64_t n,
                 int ncb, int nrb, int nks, int upk, float *__restrict__ ws) {
   constexpr int SB = ScaleTraits<KIND>::bytes;
@@ -222,7 +220,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
   constexpr int LPR = 4 * PU, RPI = 64 / LPR;          // lanes per row, rows per load of codes
   constexpr int WL = 32 / RPI;                         // loads of codes per column tile
   static_assert(XF % KW == 0 && PU * UB % 4 == 0, "whole fragments and scale dwords");
-  __shared__ f16x8 xs[2][XF][64];
+  __shared__ bf16x8_t xs[2][XF][64];
   __shared__ __attribute__((aligned(16))) int exs[32 * RT];
   __shared__ __attribute__((aligned(16))) uint8_t cl[KW][32][PU * kUnit + 16];
 
@@ -260,7 +258,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
   // the fragments this wave stages: numbers wid + KW i of the phase's XF
   // (unit, row tile, fragment)
   const int ntile = (s + 31) / 32;
-  const _Float16 *xt[XL];                              // (uniform: scalar base, lane offset)
+  const __bf16 *xt[XL];                              // (uniform: scalar base, lane offset)
   int xun[XL];                                         // unit of the phase
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
@@ -272,7 +270,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
 
   const uint32_t lane16 = 16u * lane;
   u32x4 W[2][WL];
-  f16x8 X[2][XL];
+  bf16x8_t X[2][XL];
   Dwords<SD> SC[2];
   // Units past u1 take the unit of zeros behind the row of x and reread the
   // codes of the last unit, and a last unit of 32 codes reads its first
@@ -286,7 +284,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
       const int u = up + xun[i] < u1 ? up + xun[i] : nu;
-      X[st][i] = *reinterpret_cast<const f16x8 *>(
+      X[st][i] = *reinterpret_cast<const bf16x8_t *>(
           reinterpret_cast<const uint8_t *>(xt[i] + (int64_t)u * (XU * 512)) + (lane16 & on));
     }
     const int us = up < u1 ? up : u1 - 1;
@@ -314,74 +312,65 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
     for (int v = 0; v < 16; ++v) acc[t][v] = 0.0f;
 
   // The PU RT blocks (unit up + v, row tile t) of a phase, from register
-  // stage and x buffer st.  A block's fragments are read from LDS one block
-  // ahead, and its partials are folded into the output behind the MFMAs of
-  // the next block.  Nothing is skipped: units past u1 and groups past m met
-  // zeros of x, and their scale is forced to 0.
+  // stage and x buffer st, as a chain of 4-step blocks.  The fragments of a
+  // step are read from LDS AH steps ahead (with three terms two or three steps
+  // spill: 200 x 1600 x 4800 32.3 -> 32.7 and 33.6 us), and a group's
+  // partials are folded into the output behind the MFMAs of the next group.
+  // Nothing is skipped: units past u1 and groups past m met zeros of x,
+  // and their scale is forced to 0.
   auto compute = [&](int st, int up, const Dwords<SD> &scd) {
-    constexpr int NB = PU * RT;
-    f16x8 a[2][XU], b[4];
+    constexpr int NX = 4 * PU * RT, AH = NT == 1 ? 4 : 1;
+    bf16x8_t a[AH + 1][NT], b[4];
     u32x4 q[2][2];
-    // (two groups per unit: their partials already fill the registers that
-    // a second set would take)
-    constexpr int DB = GPU_ == 1 ? 2 : 1;
-    f32x16 d[DB][GPU_];
-    auto read_a = [&](int blk) {
+    f32x16 d[2];
+    auto read_a = [&](int x) {
 #pragma unroll
-      for (int i = 0; i < XU; ++i) a[blk & 1][i] = xs[st][blk * XU + i][lane];
-      if (blk % RT == 0) {
-        const int v = blk / RT;
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-          q[v & 1][p] = *reinterpret_cast<const u32x4 *>(
-              &cl[wid][lr][kUnit * v + (G == 64 ? 32 * lh + 16 * p : 32 * p + 16 * lh)]);
-      }
+      for (int t = 0; t < NT; ++t) a[x % (AH + 1)][t] = xs[st][x * NT + t][lane];
     };
-    auto fold = [&](int blk) {
-      const int v = blk / RT, t = blk % RT;
+    auto read_q = [&](int v) {
 #pragma unroll
-      for (int g = 0; g < GPU_; ++g) {
-        const bool live = up + v < u1 && (up + v) * kUnit + g * G < m;
-        const int byte = v * UB + g * SB;
-        const uint32_t raw = scd.d[byte >> 2];
-        float sc = KIND == SCALE_F16 ? f16_bits_to_f32((uint16_t)(raw >> (8 * (byte & 3))))
-                                     : __builtin_bit_cast(float, raw);
-        sc = live ? sc : 0.0f;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[t][e] = __builtin_fmaf(sc, d[blk % DB][g][e], acc[t][e]);
-      }
+      for (int p = 0; p < 2; ++p)
+        q[v & 1][p] = *reinterpret_cast<const u32x4 *>(
+            &cl[wid][lr][kUnit * v + (G == 64 ? 32 * lh + 16 * p : 32 * p + 16 * lh)]);
     };
-    read_a(0);
+    auto fold = [&](int j) {                   // group j of the chain
+      const int blk = j / GPU_, g = j % GPU_, v = blk / RT, t = blk % RT;
+      const bool live = up + v < u1 && (up + v) * kUnit + g * G < m;
+      const int byte = v * UB + g * SB;
+      const uint32_t raw = scd.d[byte >> 2];
+      float sc = KIND == SCALE_F16 ? f16_bits_to_f32((uint16_t)(raw >> (8 * (byte & 3))))
+                                   : __builtin_bit_cast(float, raw);
+      sc = live ? sc : 0.0f;
 #pragma unroll
-    for (int blk = 0; blk < NB; ++blk) {
-      const int v = blk / RT;
-      if (blk + 1 < NB) read_a(blk + 1);
+      for (int e = 0; e < 16; ++e) acc[t][e] = __builtin_fmaf(sc, d[j & 1][e], acc[t][e]);
+    };
+    read_q(0);
+#pragma unroll
+    for (int x = 0; x < AH; ++x) read_a(x);
+#pragma unroll
+    for (int x = 0; x < NX; ++x) {
+      const int step = x % 4, blk = x / 4, v = blk / RT, j = x / SPG;
+      if (x + AH < NX) read_a(x + AH);
+      if (step == 0 && blk % RT == RT - 1 && v + 1 < PU) read_q(v + 1);
       __builtin_amdgcn_sched_barrier(0);
-      if (blk % RT == 0) {                     // the unit's codes, step 2 p + e
+      if (step == 0 && blk % RT == 0) {        // the unit's codes, step 2 p + e
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-          b[2 * p] = codes_to_f16(q[v & 1][p].x, q[v & 1][p].y);
-          b[2 * p + 1] = codes_to_f16(q[v & 1][p].z, q[v & 1][p].w);
+          b[2 * p] = codes_to_bf16(q[v & 1][p].x, q[v & 1][p].y);
+          b[2 * p + 1] = codes_to_bf16(q[v & 1][p].z, q[v & 1][p].w);
         }
       }
 #pragma unroll
-      for (int i = 0; i < SPG; ++i)
+      for (int t = 0; t < NT; ++t) {
+        f32x16 z;
 #pragma unroll
-        for (int term = 0; term < NT; ++term)
-#pragma unroll
-          for (int g = 0; g < GPU_; ++g) {
-            f32x16 z;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) z[e] = 0.0f;
-            const int step = g * SPG + i;
-            d[blk % DB][g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                a[blk & 1][step * NT + term], b[step],
-                i == 0 && term == 0 ? z : d[blk % DB][g], 0, 0, 0);
-          }
-      if (DB == 1) fold(blk);
-      if (DB == 2 && blk > 0) fold(blk - 1);
+        for (int e = 0; e < 16; ++e) z[e] = 0.0f;
+        d[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            a[x % (AH + 1)][t], b[step], x % SPG == 0 && t == 0 ? z : d[j & 1], 0, 0, 0);
+      }
+      if (x % SPG == SPG - 1 && j > 0) fold(j - 1);
     }
-    if (DB == 2) fold(NB - 1);
+    fold(NX / SPG - 1);
   };
 
   // Phase p loads phase p + 2 into register stage p & 1 (stored to LDS in
@@ -428,7 +417,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const _Float16
 }
 
 template <int G, int KIND, int NT, int RT, int KW>
-hipError_t launch_t(const LinearArgs &a, const _Float16 *xf, const int *ex, hipStream_t st) {
+hipError_t launch_t(const LinearArgs &a, const __bf16 *xf, const int *ex, hipStream_t st) {
   const int64_t ncb = (a.n + 32 * KW - 1) / (32 * KW), nrb = (a.s + 32 * RT - 1) / (32 * RT);
   const int nu = (int)((a.m + kUnit - 1) / kUnit);
   int nks = 1;
@@ -447,22 +436,22 @@ hipError_t launch_t(const LinearArgs &a, const _Float16 *xf, const int *ex, hipS
 }
 
 template <int G, int KIND>
-hipError_t launch_g(const LinearArgs &a, _Float16 *xf, int *ex, hipStream_t st) {
+hipError_t launch_g(const LinearArgs &a, __bf16 *xf, int *ex, hipStream_t st) {
   if (a.x_is_bf16) {
-    launch_frag16<false, 1, G>(a, xf, ex, st);
+    launch_frag<false, 1, G>(a, xf, ex, st);
     if (a.s <= 32) return launch_t<G, KIND, 1, 1, 4>(a, xf, ex, st);
     return launch_t<G, KIND, 1, 2, 8>(a, xf, ex, st);
   }
-  launch_frag16<true, 2, G>(a, xf, ex, st);
-  if (a.s <= 32) return launch_t<G, KIND, 2, 1, 4>(a, xf, ex, st);
-  return launch_t<G, KIND, 2, 2, 8>(a, xf, ex, st);
+  launch_frag<true, 3, G>(a, xf, ex, st);
+  if (a.s <= 32) return launch_t<G, KIND, 3, 1, 4>(a, xf, ex, st);
+  return launch_t<G, KIND, 3, 2, 8>(a, xf, ex, st);
 }
 
 }  // namespace
 
 int64_t mid_rows(int64_t bytes, int64_t m, bool x_is_bf16) {
   const int64_t nu = (m + kUnit - 1) / kUnit;
-  const int64_t tile = (nu + 1) * kUnit * 32 * (x_is_bf16 ? 2 : 4) + 32 * 4;
+  const int64_t tile = (nu + 1) * kUnit * 32 * (x_is_bf16 ? 2 : 6) + 32 * 4;
   return bytes / tile * 32;
 }
 
@@ -477,8 +466,9 @@ hipError_t launch_mid(const LinearArgs &a, void *scratch, int64_t bytes, hipStre
     la.s = s - r0 < rows ? s - r0 : rows;
     la.x = static_cast<const uint8_t *>(a.x) + r0 * a.m * xb;
     la.y = a.y + r0 * a.n;
-    _Float16 *xf = static_cast<_Float16 *>(scratch);
-    int *ex = reinterpret_cast<int *>(static_cast<uint8_t *>(scratch) + rows * (nu + 1) * kUnit * xb);
+    __bf16 *xf = static_cast<__bf16 *>(scratch);
+    int *ex = reinterpret_cast<int *>(static_cast<uint8_t *>(scratch) +
+                                      rows * (nu + 1) * kUnit * (a.x_is_bf16 ? 2 : 6));
     hipError_t e = hipErrorInvalidValue;
     if (a.G == 64 && a.kind == SCALE_F16) e = launch_g<64, SCALE_F16>(la, xf, ex, st);
     if (a.G == 64 && a.kind == SCALE_F32) e = launch_g<64, SCALE_F32>(la, xf, ex, st);

@@ -486,10 +486,9 @@ constexpr int64_t kGemmMinRows = 32;
 // 17 .. 31 rows of at least this many codes take the fragment MFMA path,
 // which reads each code once per 32 rows; on shorter rows its two extra
 // launches cost more than that saves (17 and 31 rows, small-batch kernel ->
-// fragments: 4096 x 6144 23.1 / 32.7 -> 17.4 / 18.2 us, 4096 x 24576 55.0 /
-// 64.6 -> 43.3 / 44.0, 12288 x 4096 33.2 -> 23.8 at 17, 8192 x 2048 22.9 /
-// 32.3 -> 16.2 / 17.9; but 2048 x 16384 16.4 / 21.0 -> 17.4 / 18.2, 1024 x
-// 6144 7.8 / 10.3 -> 11.0 / 12.0).
+// fragments: 4096 x 6144 23.1 / 32.7 -> 18.8 / 19.9 us, 4096 x 24576 55.0 /
+// 64.6 -> 43.6 / 44.5, 14336 x 4096 38.0 / 52.8 -> 31.0 / 33.3, 8192 x 2048
+// 22.8 / 32.4 -> 17.1 / 19.0).
 constexpr int64_t kMidMinWidth = 4096;
 
 // Attach the context's split-K workspace to a launch.

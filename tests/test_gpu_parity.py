@@ -323,7 +323,7 @@ UNALIGNED = [(1, 96, 7), (1, 1600, 333), (1, 4160, 4100), (1, 1600, 9000), (1, 6
 def test_linear_any_alignment(ctx, cor, G, scale, s, m, n, act):
     """Packed rows at an offset of 3 u16, whose lengths are mostly no
     multiple of 16 bytes, and x one element off: one row on the GEMV,
-    more rows (and bf16 x) as binary16 fragments on the matrix cores, every
+    more rows (and bf16 x) as bf16 fragments on the matrix cores, every
     product exact in f32.  Bar: the f32 sums of a row, at most m / 32 group
     partials of 32 products each, stay within (m / 32 + 32) 2^-24 of
     float64 normwise (7.5e-5 at m = 40032); 1e-5 is asked below that."""
@@ -412,6 +412,39 @@ def test_linear_unaligned_infinities_and_tiny_rows(ctx, cor):
         with np.errstate(invalid="ignore"):
             want = sign * np.float32(np.inf) * q
         assert np.array_equal(y[b], want, equal_nan=True), b
+
+
+@pytest.mark.parametrize("G,scale", LAYOUTS)
+@pytest.mark.parametrize("s,m,n,off,act", [(20, 4096, 1500, 0, "f32"), (200, 1600, 300, 3, "f32"),
+                                           (40, 11008, 65, 1, "f32"), (200, 1600, 300, 3, "bf16"),
+                                           (1, 11008, 65, 1, "bf16")])
+def test_linear_carries_x_beside_a_large_channel(ctx, cor, G, scale, s, m, n, off, act):
+    """x is carried exactly, not to a share of its row's largest value: one
+    channel is 2^34 times the others, and half of the outputs have a code of
+    0 there.  Their error is that of the f32 sums of the rest (1e-5 of each
+    output's own sum of absolute products, as above)."""
+    say("large channel", G, scale, s, m, n, off, act)
+    rng = np.random.default_rng(m + n)
+    wf = (rng.standard_normal((n, m)) * 0.02).astype(np.float32)
+    wf[::2, 77] = 0.0
+    pk = cor.pack_f32(wf, G, scale)
+    x = synth_x(s, m, seed=9)
+    x[:, 77] = 2.0 ** 34
+    if act == "bf16":
+        xbits = f32_to_bf16_bits(x)
+        w = upload(ctx, np.concatenate([np.zeros(off, np.uint16), pk.reshape(-1)]))
+        xb = upload(ctx, xbits)
+        yb = ctx.alloc(4 * s * n)
+        q8hip.linear_bf16act(ctx, w, off, xb, 0, yb, 0, s, m, n, G, scale)
+        y = yb.download((s, n), np.float32)
+        for buf in (w, xb, yb):
+            buf.free()
+        x = bf16_bits_to_f32(xbits)
+    else:
+        y = gpu_linear(ctx, pk, x, G, scale, owt=off)
+    ref, size = cor.linear_f64(pk, x, G, scale), cor.linear_abs(pk, x, G, scale)
+    assert elementwise_err(y, ref, size) <= 1e-5
+    assert np.abs(ref[:, ::2]).max() < 1e-6 * np.abs(ref[:, 1::2]).max()
 
 
 def test_linear_unaligned_rows_past_the_scratch(cor):
