@@ -155,7 +155,8 @@ int q8_linear_bf16act(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *x,
  * need no context.  y[s, n] = x[s, m] . deq(W[n, m])^T exactly as q8_linear
  * computes it (same kernels and split decisions, so the same bits, except
  * from s = 32 on when the rows do not fit the 16 MiB activation buffer at
- * once: they then run in chunks, within the same 1e-3 contract), on
+ * once: they then run in chunks, or unaligned rows of more than 87296 values
+ * one output per wave, within the same 1e-3 contract), on
  * hip_stream (NULL: the null stream), which must belong to the current
  * device.  w points at packed row 0 (rows back to back) and must be 2-byte
  * aligned; x and y are f32, 4-byte aligned, and must not overlap (else
@@ -163,8 +164,8 @@ int q8_linear_bf16act(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *x,
  * Scratch: one fixed __device__ array of Q8_NOALLOC_SCRATCH_BYTES (32 MiB)
  * per GPU, resident on every GPU where the library's code object is loaded
  * until the process ends, used or not (16 MiB of split-K partials and a
- * 16 MiB binary16 activation buffer for s >= 32, which takes the rows in
- * chunks).
+ * 16 MiB activation buffer: binary16 rows for s >= 32, in chunks; bf16
+ * fragments of 17 .. 31 rows and of unaligned ones from two rows on).
  * Limit: from s = 32 on, one activation row (2 m + 4 bytes) plus 4 n bytes
  * must fit in 16 MiB, else Q8_ERR_SHAPE.  Every call on a GPU shares that
  * GPU's array: calls that overlap on one GPU (two streams, two threads)

@@ -25,7 +25,7 @@
 // + m bytes, so most widths that are no multiple of 512 at G = 64 with f16
 // scales), against one wave per output with one code per lane and load:
 // 200 x 1600 x 4800 1030 -> 32 us, 512 x 11008 x 4096 24390 -> 166 us, 20 x
-// 11008 x 4096 970 -> 28 us; and 17 .. 31
+// 11008 x 4096 960 -> 28 us; and 17 .. 31
 // aligned rows of 4096 codes or more (31 x 4096 x 24576 65 -> 45 us; the line
 // is drawn in the dispatch).
 //

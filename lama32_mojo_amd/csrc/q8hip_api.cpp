@@ -9,6 +9,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -552,11 +553,20 @@ struct Scratch {
   int64_t act_bytes;
 };
 
+// Bytes of fragments that decide whether a row is short enough for the
+// fragment path: below kGemmMinRows rows the smaller activation buffer's
+// whatever the call's own is, since q8_linear and q8_linear_noalloc promise
+// the same bits there (rows of up to 87296 f32 values).
+constexpr int64_t kNoAllocAct16Bytes = (int64_t)16 << 20;
+bool fragments_fit(const q8::LinearArgs &la, int64_t bytes) {
+  return q8::mid_rows(la.s < kGemmMinRows ? std::min(bytes, kNoAllocAct16Bytes) : bytes, la.m,
+                      la.x_is_bf16) > 0;
+}
+
 // Operands that are not 16-byte aligned, two rows and up or bf16 x: the
-// fragment MFMA path; the generic GEMV when a tile of 32 rows does not fit
-// the activation buffer (rows of 500 thousand values in 64 MiB).
+// fragment MFMA path; the generic GEMV when a tile of 32 rows does not fit.
 hipError_t run_unaligned(const q8::LinearArgs &la, void *act16, int64_t bytes, hipStream_t st) {
-  if (q8::mid_rows(bytes, la.m, la.x_is_bf16) > 0) return q8::launch_mid(la, act16, bytes, st);
+  if (fragments_fit(la, bytes)) return q8::launch_mid(la, act16, bytes, st);
   return q8::launch_gemv(la, st);
 }
 
@@ -570,7 +580,7 @@ hipError_t dispatch_linear(q8::LinearArgs la, const Scratch &sc, hipStream_t st)
   if (!gemm_aligned(la)) return run_unaligned(la, sc.act16, sc.act_bytes, st);
   if (la.s >= kGemmMinRows) return run_gemm_in(la, sc.act16, sc.act_bytes, st);
   if (la.s <= q8::kSkinny4MaxRows) return q8::launch_skinny4(la, st);
-  if (la.s > 16 && la.m >= kMidMinWidth && q8::mid_rows(sc.act_bytes, la.m, 0) > 0)
+  if (la.s > 16 && la.m >= kMidMinWidth && fragments_fit(la, sc.act_bytes))
     return q8::launch_mid(la, sc.act16, sc.act_bytes, st);
   return q8::launch_skinny(la, st);
 }
@@ -672,15 +682,14 @@ int q8_linear_bf16act(q8_ctx *ctx, q8_buf *w, uint64_t owt_u16, q8_buf *x, uint6
 // q8_linear_noalloc keeps its scratch in one fixed device array per GPU
 // instead of a context's workspace: 16 MiB of split-K partial sums (the size
 // of a context's, so it makes the same split decisions as q8_linear), then
-// the GEMM's 16 MiB binary16 activation buffer.  The array's name is a host-side stand-in: host code
-// only ever passes the address hipGetSymbolAddress returns for the current
-// device (noalloc_scratch).
+// a 16 MiB activation buffer (the GEMM's binary16 rows, or fragments).  The
+// array's name is a host-side stand-in: host code only ever passes the
+// address hipGetSymbolAddress returns for the current device
+// (noalloc_scratch).
 
 namespace {
 constexpr int64_t kNoAllocWsFloats = kGemmWsFloats;
-constexpr int64_t kNoAllocAct16Bytes = (int64_t)16 << 20;
-constexpr int64_t kNoAllocBytes =
-    kNoAllocWsFloats * 4 + kNoAllocAct16Bytes;
+constexpr int64_t kNoAllocBytes = kNoAllocWsFloats * 4 + kNoAllocAct16Bytes;
 static_assert(kNoAllocBytes == Q8_NOALLOC_SCRATCH_BYTES, "scratch size differs from the header");
 }  // namespace
 

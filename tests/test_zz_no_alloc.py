@@ -72,6 +72,61 @@ def test_noalloc_equals_q8_linear(ctx, cor, G, scale, first, second, path):
         a.free()
 
 
+# (s, n, m, w and x offsets in elements): 17 to 31 rows of 4096 codes and more,
+# unaligned rows, and rows of either kind too long for 16 MiB of fragments but
+# not for a context's 64 MiB
+FRAGMENTS = [(17, 2500, 4096, 0, 0), (31, 1000, 8192, 0, 0), (2, 9000, 1632, 3, 1),
+             (31, 4100, 1632, 0, 0), (5, 2100, 11008, 1, 0), (17, 24, 90112, 0, 0), (17, 8, 131072, 0, 0),
+             (31, 5, 87296, 1, 1), (2, 5, 87328, 1, 1), (6, 3, 131104, 0, 0)]
+
+
+@pytest.mark.parametrize("scale", ["f16", "f32"])
+@pytest.mark.parametrize("s,n,m,ow,ox", FRAGMENTS)
+def test_noalloc_equals_q8_linear_below_32_rows(ctx, cor, scale, s, n, m, ow, ox):
+    """The route of a call below 32 rows does not depend on whose scratch it
+    has: the same bits eagerly and on every replay of a captured call, with
+    other uses of the scratch in between, within 1e-5 of float64 (2e-5 where
+    rows of 87 thousand values and more are summed)."""
+    say("noalloc below 32 rows", scale, s, n, m, ow, ox)
+    G = 32
+    pk = cor.pack_bf16(synth_weights_bf16(n, m, seed=n + s), G, scale)
+    w = ctx.alloc(pk.nbytes + 2 * ow)
+    w.upload(pk, 2 * ow)
+    x = synth_x(s, m, seed=s + 1)
+    a = ctx.alloc(4 * (ox + s * m + 2 * s * n))
+    a.upload(x, 4 * ox)
+    o1 = ox + s * m
+    o2 = o1 + s * n
+
+    def noalloc():
+        q8hip.linear_noalloc(ctx.stream, w.ptr + 2 * ow, a.ptr + 4 * ox, a.ptr + 4 * o2, s, m, n, G,
+                             scale)
+
+    q8hip.linear(ctx, w, ow, a, ox, o1, s, m, n, G, scale)
+    noalloc()
+    ctx.sync()
+    want = a.download((s, n), np.float32, 4 * o1)
+    assert np.array_equal(a.download((s, n), np.float32, 4 * o2), want)
+    assert max_rel_err(want, cor.linear_f64(pk, x, G, scale)) <= (1e-5 if m < 87000 else 2e-5)
+    other = case_buffers(ctx, cor, 64, 512, 1024, G, scale, seed=5)
+    ctx.graph_begin()
+    try:
+        noalloc()
+    finally:
+        g = ctx.graph_end()
+    try:
+        for rep in range(3):
+            a.upload(np.full((s, n), np.nan, np.float32), 4 * o2)
+            run_both(ctx, other[1], other[3], 64, 1024, 512, G, scale)
+            g.launch()
+            ctx.sync()
+            assert np.array_equal(a.download((s, n), np.float32, 4 * o2), want), rep
+    finally:
+        g.destroy()
+        for b in (w, a, other[1], other[3]):
+            b.free()
+
+
 def test_noalloc_gemm_in_row_chunks(ctx, cor):
     """1024 rows of 8192 binary16 values (16 MiB) do not fit the 16 MiB
     activation buffer with the weight exponents: two row chunks, each its
