@@ -399,8 +399,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(
 }
 
 // Any alignment, row count and activation dtype: one wavefront per output,
-// one code per lane per step.  Only for rows too long for the fragment
-// scratch of the MFMA path (launch_mid).
+// one code per lane per step.  For little work, where one launch is all that
+// counts, and rows too long for the fragment scratch of the MFMA path
+// (launch_mid).
 template <int G, int KIND, bool XBF16>
 __global__ __launch_bounds__(256) void gemv_generic_kernel(
     const uint8_t *__restrict__ w, int64_t row_bytes, int64_t n,

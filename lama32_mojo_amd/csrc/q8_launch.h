@@ -47,8 +47,8 @@ struct LinearArgs {
   const float *res = nullptr;
   float *hout = nullptr;
 };
-// Decode path (s = 1, f32 x, any alignment): VALU GEMV; more rows only as the
-// last resort of unaligned operands that fit no scratch.
+// Decode path (s = 1, f32 x, any alignment): VALU GEMV; more rows only of
+// unaligned operands, few products or rows that fit no scratch.
 hipError_t launch_gemv(const LinearArgs &a, hipStream_t st);
 // One-row GEMV with its neighbours folded in (decode step, s = 1).
 // Prologue (how x is read):

@@ -563,10 +563,27 @@ bool fragments_fit(const q8::LinearArgs &la, int64_t bytes) {
                       la.x_is_bf16) > 0;
 }
 
+// Unaligned operands with so little work that the generic GEMV's one launch
+// (2 us, 0.17-0.2 us per group of a row, and 0.5 us per million products at
+// G = 64, 1.4 at G = 32) is over before the fragments' two or three (f32 x
+// 8 us below 512 codes and 12-14 above, bf16 x 7.5 and 10.5-12.5): rows of up
+// to 50 groups and this many products.  Generic and fragments, us: 16 x 576 x
+// 1024 (9 M products) G64 8.0 and 13.5, 16 x 1600 x 512 (13 M) 9.1 and 13.5,
+// 2 x 1600 x 4800 (15 M) 13.0 and 13.5, 32 x 1600 x 512 (26 M) 16.1 and 14.0;
+// G32 8 x 576 x 1024 (5 M) 8.6 and 14.2, 16 x 576 x 1024 (9 M) 15.3 and 14.4;
+// bf16 x at G64 1 x 1600 x 4800 8.0 and 11.0, 2 x 1600 x 4800 13.1 and 11.3;
+// 51 groups and up 2 x 11008 x 64 33.3 and 14.9.
+bool few_products(const q8::LinearArgs &la) {
+  const int64_t most = la.G == 64 ? (la.x_is_bf16 ? 14000000 : 18000000)
+                                  : (la.x_is_bf16 ? 5000000 : 7000000);
+  return la.m <= 50 * la.G && la.s * la.n <= most / la.m;
+}
+
 // Operands that are not 16-byte aligned, two rows and up or bf16 x: the
-// fragment MFMA path; the generic GEMV when a tile of 32 rows does not fit.
+// fragment MFMA path; the generic GEMV for little work, and when a tile of 32
+// rows does not fit.
 hipError_t run_unaligned(const q8::LinearArgs &la, void *act16, int64_t bytes, hipStream_t st) {
-  if (fragments_fit(la, bytes)) return q8::launch_mid(la, act16, bytes, st);
+  if (!few_products(la) && fragments_fit(la, bytes)) return q8::launch_mid(la, act16, bytes, st);
   return q8::launch_gemv(la, st);
 }
 

@@ -323,8 +323,8 @@ UNALIGNED = [(1, 96, 7), (1, 1600, 333), (1, 4160, 4100), (1, 1600, 9000), (1, 6
 def test_linear_any_alignment(ctx, cor, G, scale, s, m, n, act):
     """Packed rows at an offset of 3 u16, whose lengths are mostly no
     multiple of 16 bytes, and x one element off: one row on the GEMV,
-    more rows (and bf16 x) as bf16 fragments on the matrix cores, every
-    product exact in f32.  Bar: the f32 sums of a row, at most m / 32 group
+    more rows (and bf16 x) on the generic GEMV or as bf16 fragments on the
+    matrix cores, every product exact in f32.  Bar: the f32 sums of a row, at most m / 32 group
     partials of 32 products each, stay within (m / 32 + 32) 2^-24 of
     float64 normwise (7.5e-5 at m = 40032); 1e-5 is asked below that."""
     if m % G:
@@ -348,6 +348,25 @@ def test_linear_any_alignment(ctx, cor, G, scale, s, m, n, act):
     for b in range(s):
         assert max_rel_err(y[b], ref[b]) <= 1e-5, b
     assert elementwise_err(y, ref, cor.linear_abs(pk, x, G, scale)) <= 1e-5
+
+
+# (s, m, n) of the fragment path: rows of more than 50 groups around its
+# tiles of 32 rows and 32, 128 and 256 columns, with a last unit of 32 codes at
+# G = 32, and products on either side of the generic GEMV's limits (G64 18 M,
+# bf16 x 14 M; G32 7 M, 5 M)
+FRAGMENTS = [(1, 3264, 130), (2, 3232, 1), (5, 3264, 31), (31, 3232, 129), (32, 3264, 333),
+             (33, 3232, 257), (65, 3264, 100), (200, 3264, 300), (16, 1600, 703), (16, 1600, 704),
+             (16, 1600, 546), (16, 1600, 547), (16, 1600, 273), (16, 1600, 274), (16, 1600, 195),
+             (16, 1600, 196), (3, 1632, 4800)]
+
+
+@pytest.mark.parametrize("G,scale", LAYOUTS + [(32, "f16"), (64, "f32")])
+@pytest.mark.parametrize("s,m,n", FRAGMENTS)
+@pytest.mark.parametrize("act", ["f32", "bf16"])
+def test_linear_fragments_any_alignment(ctx, cor, G, scale, s, m, n, act):
+    """The sizes of the fragment path and of the line to the generic GEMV, held
+    to the bars of test_linear_any_alignment."""
+    test_linear_any_alignment(ctx, cor, G, scale, s, m, n, act)
 
 
 @pytest.mark.parametrize("G,scale,s,m,n", [
