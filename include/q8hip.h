@@ -127,7 +127,7 @@ int q8_quantize_pack(q8_ctx *ctx, q8_buf *src, uint64_t src_off, int src_dtype,
  * codes; 5 .. 31 rows split each x into two bf16 terms hi + lo (x - hi - lo
  * below 2^-17 |x|, so x is carried to that bound, not exactly) whose
  * products with the codes are exact on bf16 MFMA; 17 .. 31 rows of m >= 4096
- * codes, and two rows and up whose packed rows or x are not 16-byte aligned,
+ * codes (but for some n), and two rows and up whose packed rows or x are not 16-byte aligned,
  * carry x as three bf16 terms whose sum is x, again with exact products
  * (little work of the latter kind runs in f32); all of these stay within 1e-5
  * of float64.  s >= 32 runs the dequant-GEMM on f16 MFMA (binary16 x

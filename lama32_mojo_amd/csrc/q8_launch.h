@@ -91,7 +91,7 @@ hipError_t launch_gemm(const LinearArgs &a, uint16_t *x16, int *ex, int *ew, boo
 hipError_t launch_splitk_reduce(const float *ws, float *y, int64_t count, int splits,
                                 hipStream_t st);
 // Small batches (s <= 32, f32 x; the C ABI sends it 5 <= s < 32, from 17 rows
-// on only where a row has fewer than 4096 codes or fits no scratch): bf16 MFMA
+// on only where the fragment path does not pay): bf16 MFMA
 // over zero-padded 16-row tiles with x split into two bf16 terms.
 hipError_t launch_skinny(const LinearArgs &a, hipStream_t st);
 // A few rows (2 <= s <= kSkinny4MaxRows, f32 x): f32 4x4 MFMA blocks over

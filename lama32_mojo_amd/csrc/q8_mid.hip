@@ -26,7 +26,7 @@
 // scales) with more than a few products, against one wave per output with one code per lane and load:
 // 200 x 1600 x 4800 1030 -> 32 us, 512 x 11008 x 4096 24390 -> 166 us, 20 x
 // 11008 x 4096 960 -> 28 us; and 17 .. 31
-// aligned rows of 4096 codes or more (31 x 4096 x 24576 65 -> 45 us); both
+// aligned rows of 4096 codes or more, but for some n (31 x 4096 x 24576 65 -> 45 us); both
 // lines are drawn in the dispatch.
 //
 // Layout: a workgroup owns 32 RT rows x 32 KW columns, wave w 32 columns of

@@ -1,6 +1,6 @@
 // q8_skinny.hip -- decode-path Q8 linear for small batches (5 <= s < 32,
-// aligned f32 activations; 17 rows and up of 4096 codes or more take
-// q8_mid.hip) on gfx950 bf16 MFMA.
+// aligned f32 activations; 17 rows and up of 4096 codes or more mostly
+// take q8_mid.hip) on gfx950 bf16 MFMA.
 //
 // y[b, j] = sum_g scale[j, g] * sum_{k in g} x[b, k] * q[j, k]
 // (k_mm_q8, src/llama_q8.mojo:54-93: unscaled dot per group, then one scale

@@ -484,13 +484,27 @@ bool gemm_aligned(const q8::LinearArgs &a) {
 // on f16 MFMA.
 constexpr int64_t kSkinnyMinRows = 2;
 constexpr int64_t kGemmMinRows = 32;
-// 17 .. 31 rows of at least this many codes take the fragment MFMA path,
-// which reads each code once per 32 rows; on shorter rows its two extra
-// launches cost more than that saves (17 and 31 rows, small-batch kernel ->
-// fragments: 4096 x 6144 23.1 / 32.7 -> 18.8 / 19.9 us, 4096 x 24576 55.0 /
-// 64.6 -> 43.6 / 44.5, 14336 x 4096 38.0 / 52.8 -> 31.0 / 33.3, 8192 x 2048
-// 22.8 / 32.4 -> 17.1 / 19.0).
-constexpr int64_t kMidMinWidth = 4096;
+// 17 .. 31 aligned rows on the fragment MFMA path, which reads each code once
+// per 32 rows, in place of the small-batch kernel, whose time grows with the
+// rows: from 4096 codes a row on, below which the two extra launches cost
+// more than that saves, with these exceptions (small-batch kernel and
+// fragments, us):
+//   - vocabulary heads, where the small-batch kernel has workgroups of 256
+//     outputs and 32 rows: 17 / 31 x 4096 x 128256 131 / 140 and 165 / 169;
+//   - its grid of one workgroup per CU: 17 / 20 / 24 x 4096 x 4096 12.3 / 13.7 /
+//     15.1 and 15.2 / 15.6 / 15.9, x 3072 13.0 / 14.5 / 15.9 and 14.6 / 14.9 /
+//     15.2, 5120 x 4096 15.2 / 16.5 / 18.1 and 18.8 / 19.1 / 19.3;
+//   - G = 64, two column tiles a wave: 17 / 20 / 24 x 7168 x 24576 64 / 69 / 75
+//     and 75 / 76 / 76, x 4096 x 16384 26.5 / 29.1 / 31.7 and 28.7 / 28.9 / 29.1.
+// Elsewhere 17 / 31 rows: 4096 x 64 12.7 / 17.7 -> 11.6 / 12.2, x 1024 13.0 /
+// 18.1 -> 12.4 / 13.5, x 6144 23.1 / 32.5 -> 19.5 / 20.5, x 28672 50.5 / 67.9 ->
+// 43.9 / 44.8, 14336 x 4096 38.0 / 52.8 -> 31.0 / 33.3.
+bool fragments_pay(const q8::LinearArgs &la) {
+  if (la.s <= 16 || la.m < 4096 || la.n >= 65536) return false;
+  if (la.m < 8192 && la.n > 2048 && la.n <= 4096) return la.s >= 24;
+  if (la.G == 64 && la.m < 8192 && la.n >= 16384 && la.n <= 24576) return la.s > 20;
+  return true;
+}
 
 // Attach the context's split-K workspace to a launch.
 void attach_gemm_workspace(q8_ctx *ctx, q8::LinearArgs &la) {
@@ -597,7 +611,7 @@ hipError_t dispatch_linear(q8::LinearArgs la, const Scratch &sc, hipStream_t st)
   if (!gemm_aligned(la)) return run_unaligned(la, sc.act16, sc.act_bytes, st);
   if (la.s >= kGemmMinRows) return run_gemm_in(la, sc.act16, sc.act_bytes, st);
   if (la.s <= q8::kSkinny4MaxRows) return q8::launch_skinny4(la, st);
-  if (la.s > 16 && la.m >= kMidMinWidth && fragments_fit(la, sc.act_bytes))
+  if (fragments_pay(la) && fragments_fit(la, sc.act_bytes))
     return q8::launch_mid(la, sc.act16, sc.act_bytes, st);
   return q8::launch_skinny(la, st);
 }

@@ -395,8 +395,8 @@ def test_gemm_iteration_counts_and_ragged_tiles(ctx, cor, G, scale, s, m, n):
 @pytest.mark.parametrize("s,m,n", [(17, 4096, 33), (31, 4096, 4100), (23, 12288, 1), (16, 4096, 33),
                                    (31, 3584, 130)])
 def test_linear_17_to_31_rows(ctx, cor, G, scale, s, m, n):
-    """17 .. 31 aligned rows of 4096 codes and more take the fragment path,
-    16 rows and shorter ones the small-batch kernel: both within 1e-5."""
+    """17 .. 31 aligned rows of 4096 codes and more mostly take the fragment
+    path, 16 rows and shorter ones the small-batch kernel: both within 1e-5."""
     say("17 to 31 rows", G, scale, s, m, n)
     pk = cor.pack_bf16(synth_weights_bf16(n, m, seed=n + s), G, scale)
     x = synth_x(s, m, seed=s + m)
@@ -404,6 +404,19 @@ def test_linear_17_to_31_rows(ctx, cor, G, scale, s, m, n):
     ref = cor.linear_f64(pk, x, G, scale)
     for b in range(s):
         assert max_rel_err(y[b], ref[b]) <= 1e-5, b
+
+
+ROWS_17_TO_31 = [(23, 4096, 2048), (23, 4096, 2049), (23, 7680, 4096), (23, 8192, 2100),
+                 (24, 4096, 2049), (23, 4096, 4097), (20, 4096, 16384), (21, 4096, 16384),
+                 (20, 4096, 24577), (17, 4096, 65536)]
+
+
+@pytest.mark.parametrize("G,scale", LAYOUTS)
+@pytest.mark.parametrize("s,m,n", ROWS_17_TO_31)
+def test_linear_17_to_31_rows_lines(ctx, cor, G, scale, s, m, n):
+    """Both sides of the lines between the fragment path and the small-batch
+    kernel."""
+    test_linear_17_to_31_rows(ctx, cor, G, scale, s, m, n)
 
 
 def test_linear_unaligned_infinities_and_tiny_rows(ctx, cor):
