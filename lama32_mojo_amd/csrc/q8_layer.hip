@@ -276,10 +276,13 @@ __device__ __forceinline__ void split_f16(float a, _Float16 &hi, _Float16 &lo) {
 // Key tiles per block when nz blocks share ntiles: all of them unless
 // sharing shortens the longest chain by 6 tiles, about what the merge launch
 // costs (0.8-1.2 us a tile; 512 rows of 64-dim heads 18.2 us whole, 19.5 in
-// two; 700 rows of 128-dim heads, 11 tiles, 32.7 and 30.5).
-__host__ __device__ inline int split_tiles(int ntiles, int nz) {
+// two; 700 rows of 128-dim heads, 11 tiles, 32.7 and 30.5).  Below 16 rows
+// the merge is small and a tile takes its longest (2 us at 128 dims), so 3
+// tiles are enough: 2 rows after 255 keys 14.7 whole, 10.4 in five (13.3 by
+// the per-row kernels); 64 dims 10.0 and 8.5 (9.9).
+__host__ __device__ inline int split_tiles(int ntiles, int nz, int s) {
   const int t = (ntiles + nz - 1) / nz;
-  return ntiles - t >= 6 ? t : ntiles;
+  return ntiles - t >= (s < kPrefillMinRows ? 3 : 6) ? t : ntiles;
 }
 // One (row, head) over keys j0 .. j1-1 by one wave in f32, reading no other
 // key: o of dims lane (and lane + 64) unnormalised, with the maximum m of the
@@ -363,7 +366,7 @@ void attn_prefill_kernel(const float *__restrict__ q,
   const int ntiles = nkeys > 0 ? (nkeys + BK - 1) / BK : 0;
   // this block's tiles; with one run for all (apart == false) only block 0
   // has any
-  const int tps = SPLIT ? split_tiles(ntiles, (int)gridDim.z) : ntiles;
+  const int tps = SPLIT ? split_tiles(ntiles, (int)gridDim.z, s) : ntiles;
   const bool apart = SPLIT && tps < ntiles;
   const int kt0 = SPLIT ? (int)blockIdx.z * tps : 0;
   const int kt1 = SPLIT ? min(kt0 + tps, ntiles) : ntiles;
@@ -615,7 +618,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float *__
   const int row0 = (int)(r / nheads) / PB * PB;
   const int nkeys = min(pos0 + min(row0 + PB, s), maxlen);
   const int ntiles = nkeys > 0 ? (nkeys + kPrefillBK - 1) / kPrefillBK : 0;
-  const int tps = split_tiles(ntiles, nz);
+  const int tps = split_tiles(ntiles, nz, s);
   if (tps >= ntiles) return;
   const int64_t nz_all = nz;
   nz = (ntiles + tps - 1) / tps;                     // splits with tiles
@@ -1175,7 +1178,11 @@ hipError_t launch_attn_t(const AttnArgs &a, hipStream_t st) {
 // Key splits of the prompt-row kernel: about one block per CU in all, within
 // the scratch (512 blocks: 15 rows after 4000 20 -> 27 us).  They are
 // counted for the whole cache, so a device position gives the splits, and
-// with them the bits, of a host position.
+// with them the bits, of a host position.  There the host cannot see that a
+// context is too short to split: blocks without tiles and the merge launch
+// then cost 0.3-3 us (a cache of 2048 to 4096: 2 rows after 15 keys 8.0 -> 8.7,
+// 16 rows after 15 7.7 -> 9.9), against 30 us saved after 1000 (16 rows 42.8 ->
+// 14.1).
 template <int HD, int GRP>
 hipError_t launch_prefill_t(const AttnArgs &a, hipStream_t st) {
   constexpr int PB = 4 * (32 / GRP);
@@ -1188,7 +1195,7 @@ hipError_t launch_prefill_t(const AttnArgs &a, hipStream_t st) {
   // With the position known here: nothing to split, no merge launch.
   const int64_t keys = a.posp || a.pos0 + (int64_t)a.s > a.maxlen ? a.maxlen : a.pos0 + a.s;
   const int most = (int)((keys + kPrefillBK - 1) / kPrefillBK);
-  if (nz <= 1 || !a.ws || split_tiles(most, (int)nz) >= most) {
+  if (nz <= 1 || !a.ws || split_tiles(most, (int)nz, a.s) >= most) {
     hipLaunchKernelGGL((attn_prefill_kernel<HD, GRP, false>), dim3((unsigned)a.nkv, (unsigned)rb),
                        dim3(256), 0, st, a.q, a.kc, a.vc, a.out, nullptr, a.s, a.nheads, a.nkv,
                        a.posp, a.pos0, a.maxlen, a.ldq);
