@@ -382,6 +382,7 @@ void attn_prefill_kernel(const float *__restrict__ q,
   // q of the column: dims 16ks + 8h + 0..7, scaled by 2^e, split hi + lo
   half8 qh[KS], ql[KS];
   float cs;
+  bool tiny = false;
   {
     const float *qr = q + (int64_t)irow * ldq + head * HD + 8 * hf;
     f32x4 qv[KS][2];
@@ -407,6 +408,20 @@ void attn_prefill_kernel(const float *__restrict__ q,
         qh[k][c] = hi;
         ql[k][c] = lo;
       }
+    // The pair carries q to 2^-22, and to 2^-40 of the column's largest
+    // value.  Rows that the per-row kernels would compute in f32 are formed
+    // in f32 below where a value lies under 2^-23 of it (one ordinary column
+    // of 128 dims in 40 thousand).
+    if (s < kPrefillMinRows) {
+      uint32_t mn = ~0u;                         // (2 |q| as bits) - 1: zeros are largest
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+          mn = min(mn, (__builtin_bit_cast(uint32_t, qv[k][c >> 2][c & 3]) << 1) - 1u);
+      mn = min(mn, (uint32_t)__shfl_xor((int)mn, 32));
+      tiny = (int)(mn >> 24) + 23 < ex + 127;    // exponents
+    }
   }
 
   // staging: registers hold the next tile while the current one is used
@@ -569,7 +584,7 @@ void attn_prefill_kernel(const float *__restrict__ q,
 #pragma unroll
     for (int v = 0; v < 16; ++v) chk = __builtin_fmaf(o[t][v], 0.0f, chk);
   chk += __shfl_xor(chk, 32);
-  const bool bad = chk != 0.0f;
+  const bool bad = chk != 0.0f || tiny;
   float2 *ml = reinterpret_cast<float2 *>(part + (int64_t)gridDim.z * s * qdim);
   if (i < s && !bad) {
     const float il = apart ? 1.0f / 16384.0f : 1.0f / (l * 16384.0f);

@@ -251,6 +251,37 @@ def test_attention_non_finite_cache_rows(ctx, head_dim, nh, nkv, s, pos0):
             b.free()
 
 
+@pytest.mark.parametrize("head_dim,nh,nkv", [(128, 8, 2), (64, 4, 2)])
+@pytest.mark.parametrize("s", [1, 2, 15])
+@pytest.mark.parametrize("pos0", [20, 1500])
+@pytest.mark.parametrize("large", [2.0 ** 23, 2.0 ** 34])
+def test_attention_carries_q_beside_a_large_dim(ctx, head_dim, nh, nkv, s, pos0, large):
+    """Up to 15 rows hold q as f32 does: beside a dimension that is 2^23 or
+    2^34 times the others, and 0 in K, the scores of the others stay within
+    1e-5 (served whole and split; every second row, the others ordinary)."""
+    say("attention large q", head_dim, nh, nkv, s, pos0, large)
+    rng = np.random.default_rng(s + pos0)
+    n, qd, kvd = pos0 + s, nh * head_dim, nkv * head_dim
+    k = (rng.standard_normal((n, kvd)) * 0.7).astype(np.float16)
+    v = rng.standard_normal((n, kvd)).astype(np.float16)
+    k[:, 5::head_dim] = 0.0
+    q = rng.standard_normal((s, qd)).astype(np.float32)
+    q[::2, 5::head_dim] = large
+    kv = ctx.alloc(4 * n * kvd)
+    kv.upload(np.stack([k, v]))
+    oy = s * qd
+    a = arena(ctx, 2 * oy + q8hip.attention_scratch_floats(s, nh, head_dim, n) + 4)
+    put(a, 0, q)
+    q8hip.attention(ctx, a, 0, kv, 0, n * kvd, n, oy, 2 * oy, s, pos0, nh, nkv, head_dim)
+    got = get(a, oy, (s, qd))
+    ref = mo.attention(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), pos0, nh,
+                       nkv, head_dim)
+    for i in range(s):
+        assert max_rel_err(got[i], ref[i]) <= 1e-5, i
+    for b in (a, kv):
+        b.free()
+
+
 @pytest.mark.parametrize("head_dim,nh,nkv,s", [(64, 8, 2, 3), (128, 32, 8, 48),
                                                (64, 32, 8, 130)])
 def test_stacked_qkv_rows_equal_dense(ctx, head_dim, nh, nkv, s):
