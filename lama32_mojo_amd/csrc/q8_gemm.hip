@@ -329,7 +329,7 @@ __device__ __forceinline__ f16x8 dequant8(uint32_t d0, uint32_t d1, f16x2 s2) {
 //     a double-buffered LDS stage.
 // So the dequantizing VALU work runs beside the matrix core instead of in
 // the MFMA waves' instruction stream; one barrier per iteration hands the
-// stages over.  Tiles hold KS = 64 codes of K (128 on the 64-row tiles);
+// stages over.  Tiles hold KS = 64 or 128 codes of K (see launch_g);
 // LDS rows are padded by 16 bytes (the 16-byte fragment reads of 8
 // neighbouring rows fall on different banks).
 //
@@ -345,7 +345,7 @@ __device__ __forceinline__ f16x8 dequant8(uint32_t d0, uint32_t d1, f16x2 s2) {
 // 16-byte reads and 174 GB/s of 16-byte writes per CU here).  4 producer
 // waves instead of 8, or 3-4 register stages instead of 2, were slower or
 // equal.
-constexpr int kIterCodes = 64;     // k per iteration (128 on 64-row tiles)
+constexpr int kIterCodes = 64;     // k per iteration, where it is not 128
 constexpr int kProducerWaves = 8;
 constexpr int kStages = 2;         // register stages of the producers
 
@@ -414,8 +414,9 @@ void gemm_kernel(const uint8_t *__restrict__ w, int64_t row_bytes,
       uint32_t sc[BC];
     };
     // Loads of iteration it are unconditional: activations past m read
-    // zeros, codes past the row read bytes whose scale is forced to 0 below,
-    // and iterations past the split's range are never stored.
+    // zeros, codes past the row read bytes whose scale is forced to 0 below.
+    // Iterations past the split's range may hold the next split's values;
+    // what is stored of them is never read (below).
     auto load = [&](Stage &S, int it) {
 #pragma unroll
       for (int u = 0; u < AC; ++u) {
@@ -467,11 +468,13 @@ void gemm_kernel(const uint8_t *__restrict__ w, int64_t row_bytes,
     // iteration it: the consumers read LDS stage it & 1; write stage
     // (it + 1) & 1 (read last in iteration it - 1) from registers, which then
     // load iteration it + 1 + PD.  nit is a multiple of PD and nothing here
-    // is conditional (what is stored or loaded past the last iteration is
-    // not used): a branch or an early exit made the compiler wait for every
-    // load in flight at the head of the loop, one iteration of prefetch
-    // instead of two (64 x 6144 x 4096 17.8 -> 16.2 us, 128 x 6144 x 4096
-    // 22.0 -> 19.1; four stages are no faster).
+    // is conditional: a branch or an early exit made the compiler wait for
+    // every load in flight at the head of the loop, one iteration of
+    // prefetch instead of two (64 x 6144 x 4096 17.8 -> 16.2 us, 128 x 6144 x
+    // 4096 22.0 -> 19.1; four stages are no faster).  The last turn stores
+    // iteration nit, into stage 0 since nit is even, while the consumers read
+    // stage 1 for the last time; nothing reads stage 0 after that.
+    static_assert(PD % 2 == 0, "an even number of iterations");
     int it = 0;
     do {
 #pragma unroll
