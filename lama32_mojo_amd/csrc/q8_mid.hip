@@ -15,17 +15,17 @@
 //      codes.  |q| <= 127 is exact in bf16, so the products are exact;
 //      a group's partial starts from 0 and is folded into the output with
 //      one f32 FMA by the group's scale, as the reference does.
-// Its error is that of the f32 sums (about 1e-7 of float64).  Two binary16
+// Its error is that of the f32 sums (0.8-2e-7 of float64).  Two binary16
 // terms of a scaled row take two MFMAs instead of three and are 10-30 %
-// faster at the same error on ordinary rows (200 x 1600 x 4800 28 us against
-// 32, 512 x 11008 x 4096 127 against 166), but carry x to 2^-39 of its row's
+// faster at much the same error on ordinary rows (200 x 1600 x 4800 28 us
+// against 32.6, 512 x 11008 x 4096 127 against 172), but carry x to 2^-39 of its row's
 // largest value only: beside a channel of 2^34 the rest lost percents.
 //
 // Where it runs: rows or x that are not 16-byte aligned (a row is (m / G) SB
 // + m bytes, so most widths that are no multiple of 512 at G = 64 with f16
 // scales) with more than a few products, against one wave per output with one code per lane and load:
-// 200 x 1600 x 4800 1030 -> 32 us, 512 x 11008 x 4096 24390 -> 166 us, 20 x
-// 11008 x 4096 960 -> 28 us; and 17 .. 31
+// 200 x 1600 x 4800 1030 -> 32.6 us, 512 x 11008 x 4096 24390 -> 172 us, 20 x
+// 11008 x 4096 960 -> 29 us; and 17 .. 31
 // aligned rows of 4096 codes or more, but for some n (31 x 4096 x 24576 65 -> 45 us); both
 // lines are drawn in the dispatch.
 //
@@ -312,20 +312,23 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const __bf16 *
     for (int v = 0; v < 16; ++v) acc[t][v] = 0.0f;
 
   // The PU RT blocks (unit up + v, row tile t) of a phase, from register
-  // stage and x buffer st, as a chain of 4-step blocks.  The fragments of a
-  // step are read from LDS AH steps ahead (with three terms two or three steps
-  // spill: 200 x 1600 x 4800 32.3 -> 32.7 and 33.6 us), and a group's
+  // stage and x buffer st, as a chain of groups.  A group sums its terms from
+  // the smallest up, so that only the last of them round at the size of the
+  // sum (200 x 1600 x 4800 in order of the steps 1.13e-7 of float64, now
+  // 0.83e-7).  Fragments are read from LDS AH ahead of their MFMA (4 of three
+  // terms: 1 % slower; 6: spills), and a group's
   // partials are folded into the output behind the MFMAs of the next group.
-  // Nothing is skipped: units past u1 and groups past m met zeros of x,
-  // and their scale is forced to 0.
+  // Nothing is skipped: units past u1 and groups past m met zeros of x, and
+  // their scale is forced to 0.
   auto compute = [&](int st, int up, const Dwords<SD> &scd) {
-    constexpr int NX = 4 * PU * RT, AH = NT == 1 ? 4 : 1;
-    bf16x8_t a[AH + 1][NT], b[4];
+    constexpr int FPG = SPG * NT;              // fragments per group
+    constexpr int NG = PU * RT * GPU_, NF = NG * FPG, AH = NT == 1 ? 4 : 3;
+    bf16x8_t a[AH + 1], b[4];
     u32x4 q[2][2];
     f32x16 d[2];
-    auto read_a = [&](int x) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) a[x % (AH + 1)][t] = xs[st][x * NT + t][lane];
+    auto read_a = [&](int f) {
+      const int r = f % FPG;
+      a[f % (AH + 1)] = xs[st][(f / FPG * SPG + r % SPG) * NT + NT - 1 - r / SPG][lane];
     };
     auto read_q = [&](int v) {
 #pragma unroll
@@ -333,7 +336,7 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const __bf16 *
         q[v & 1][p] = *reinterpret_cast<const u32x4 *>(
             &cl[wid][lr][kUnit * v + (G == 64 ? 32 * lh + 16 * p : 32 * p + 16 * lh)]);
     };
-    auto fold = [&](int j) {                   // group j of the chain
+    auto fold = [&](int j) {
       const int blk = j / GPU_, g = j % GPU_, v = blk / RT, t = blk % RT;
       const bool live = up + v < u1 && (up + v) * kUnit + g * G < m;
       const int byte = v * UB + g * SB;
@@ -346,31 +349,32 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const __bf16 *
     };
     read_q(0);
 #pragma unroll
-    for (int x = 0; x < AH; ++x) read_a(x);
+    for (int f = 0; f < AH; ++f) read_a(f);
 #pragma unroll
-    for (int x = 0; x < NX; ++x) {
-      const int step = x % 4, blk = x / 4, v = blk / RT, j = x / SPG;
-      if (x + AH < NX) read_a(x + AH);
-      if (step == 0 && blk % RT == RT - 1 && v + 1 < PU) read_q(v + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      if (step == 0 && blk % RT == 0) {        // the unit's codes, step 2 p + e
+    for (int j = 0; j < NG; ++j) {
+      const int blk = j / GPU_, v = blk / RT;
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          b[2 * p] = codes_to_bf16(q[v & 1][p].x, q[v & 1][p].y);
-          b[2 * p + 1] = codes_to_bf16(q[v & 1][p].z, q[v & 1][p].w);
+      for (int r = 0; r < FPG; ++r) {
+        const int f = j * FPG + r;
+        if (f + AH < NF) read_a(f + AH);
+        if (r == 0 && j % GPU_ == 0 && blk % RT == RT - 1 && v + 1 < PU) read_q(v + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (r == 0 && j % (GPU_ * RT) == 0) {  // the unit's codes, step 2 p + e
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            b[2 * p] = codes_to_bf16(q[v & 1][p].x, q[v & 1][p].y);
+            b[2 * p + 1] = codes_to_bf16(q[v & 1][p].z, q[v & 1][p].w);
+          }
         }
-      }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
         f32x16 z;
 #pragma unroll
         for (int e = 0; e < 16; ++e) z[e] = 0.0f;
         d[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            a[x % (AH + 1)][t], b[step], x % SPG == 0 && t == 0 ? z : d[j & 1], 0, 0, 0);
+            a[f % (AH + 1)], b[j % GPU_ * SPG + r % SPG], r == 0 ? z : d[j & 1], 0, 0, 0);
       }
-      if (x % SPG == SPG - 1 && j > 0) fold(j - 1);
+      if (j > 0) fold(j - 1);
     }
-    fold(NX / SPG - 1);
+    fold(NG - 1);
   };
 
   // Phase p loads phase p + 2 into register stage p & 1 (stored to LDS in
