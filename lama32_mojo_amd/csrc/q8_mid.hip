@@ -18,16 +18,17 @@
 // Its error is that of the f32 sums (0.8-2e-7 of float64).  Two binary16
 // terms of a scaled row take two MFMAs instead of three and are 10-30 %
 // faster at much the same error on ordinary rows (200 x 1600 x 4800 28 us
-// against 32.6, 512 x 11008 x 4096 127 against 172), but carry x to 2^-39 of its row's
-// largest value only: beside a channel of 2^34 the rest lost percents.
+// against 32.6, 512 x 11008 x 4096 127 against 172), but carry x to 2^-39 of
+// its row's largest value only: beside a channel of 2^34 the rest lost
+// percents.
 //
 // Where it runs: rows or x that are not 16-byte aligned (a row is (m / G) SB
 // + m bytes, so most widths that are no multiple of 512 at G = 64 with f16
-// scales) with more than a few products, against one wave per output with one code per lane and load:
-// 200 x 1600 x 4800 1030 -> 32.6 us, 512 x 11008 x 4096 24390 -> 172 us, 20 x
-// 11008 x 4096 960 -> 29 us; and 17 .. 31
-// aligned rows of 4096 codes or more, but for some n (31 x 4096 x 24576 65 -> 45 us); both
-// lines are drawn in the dispatch.
+// scales) with more than a few products, against one wave per output with
+// one code per lane and load: 200 x 1600 x 4800 1030 -> 32.6 us, 512 x 11008 x
+// 4096 24390 -> 172 us, 20 x 11008 x 4096 960 -> 29 us; and 17 .. 31 aligned
+// rows of 4096 codes or more, but for some n (31 x 4096 x 28672 68 -> 45 us);
+// both lines are drawn in the dispatch.
 //
 // Layout: a workgroup owns 32 RT rows x 32 KW columns, wave w 32 columns of
 // them, and a range of 64-code units of K.  Per phase of two units (PU)
@@ -316,9 +317,8 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const __bf16 *
   // the smallest up, so that only the last of them round at the size of the
   // sum (200 x 1600 x 4800 in order of the steps 1.13e-7 of float64, now
   // 0.83e-7).  Fragments are read from LDS AH ahead of their MFMA (4 of three
-  // terms: 1 % slower; 6: spills), and a group's
-  // partials are folded into the output behind the MFMAs of the next group.
-  // Nothing is skipped: units past u1 and groups past m met zeros of x, and
+  // terms: 1 % slower; 6: spills), and a group's partials are folded into the
+  // output behind the MFMAs of the next group.  Nothing is skipped: units past u1 and groups past m met zeros of x, and
   // their scale is forced to 0.
   auto compute = [&](int st, int up, const Dwords<SD> &scd) {
     constexpr int FPG = SPG * NT;              // fragments per group
