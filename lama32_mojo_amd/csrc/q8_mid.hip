@@ -318,8 +318,8 @@ void mid_kernel(const uint8_t *__restrict__ w, int64_t row_bytes, const __bf16 *
   // sum (200 x 1600 x 4800 in order of the steps 1.13e-7 of float64, now
   // 0.83e-7).  Fragments are read from LDS AH ahead of their MFMA (4 of three
   // terms: 1 % slower; 6: spills), and a group's partials are folded into the
-  // output behind the MFMAs of the next group.  Nothing is skipped: units past u1 and groups past m met zeros of x, and
-  // their scale is forced to 0.
+  // output behind the MFMAs of the next group.  Nothing is skipped: units
+  // past u1 and groups past m met zeros of x, and their scale is forced to 0.
   auto compute = [&](int st, int up, const Dwords<SD> &scd) {
     constexpr int FPG = SPG * NT;              // fragments per group
     constexpr int NG = PU * RT * GPU_, NF = NG * FPG, AH = NT == 1 ? 4 : 3;
